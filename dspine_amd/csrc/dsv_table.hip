@@ -5,20 +5,26 @@
 //   msg    = gate * value                                          [R]
 //   ref    = x[n] + scale[n] * (msg @ w_last^T)                    [H]
 //   T[n, j, c] = (ref / sqrt(mean(ref^2) + eps) * norm_w) . head[n, c]
-// in float32 on the matrix cores (v_mfma_f32_16x16x4f32), three launches:
-//   k_rs_message  sender rows x R: the gathered, scaled codebook rows times [pg; pv]^T (the pg / pv
-//                 rows staged in LDS tiles shared by a workgroup's waves), with the gate, the value
-//                 and their product in the epilogue -> msg [n*K, R]
-//   k_rs_table    (row, 16 senders, H slice): msg times w_last^T (w_last staged in LDS tiles of 16
-//                 rows shared by a workgroup's four units) in 16 x 16 output blocks that are
-//                 already the B operand of the second product against the 16 candidates' head
-//                 rows, so ref never leaves registers; partial sums of ref^2 and of the dot products
+// in float32 accuracy on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16, float32 accumulation): a
+// float32 operand is three bf16 parts (split2), a bf16 operand one, and a product of two float32
+// operands is the six part products that reach float32's last bit.  Four launches:
+//   k_rs_message  sender rows x R: the gathered codebook rows times [pg; pv]^T, scaled, with the gate,
+//                 the value and their product in the epilogue -> msg's parts [n*K, 3, R]
+//   k_rs_split    w_last's parts [H, 3, R]
+//   k_rs_table    (eight units of 16 senders, H slice): msg times w_last^T in 16 x 16 output blocks
+//                 that are already the B operand of the second product against the 16 candidates'
+//                 head rows, so ref never leaves registers; partial sums of ref^2 and of the dot
+//                 products
 //   k_rs_finish   the slices combined, divided by sqrt(mean + eps)
 //
-// MFMA operand layout (16x16x4, one wave): lane l holds A[l % 16][k] and B[k][l % 16] for k of its
-// lane group g = l / 16, and receives D[4g + v][l % 16], v = 0..3.  A product of 16 k values is
-// four instructions; lane group g takes k = 4g + s at step s (a permutation of k that A and B
-// share), so every lane loads its 4 k values as one contiguous vector.
+// What bounds it: matrix-core issue and the clock under it.  n 960, K 16, H 4096, R 512, C 1024 is 92.6
+// GFLOP of float32 products, 490 GFLOP in bf16 parts: 441 us, 1.1 PFLOP/s (the library's bf16 product
+// of 8192^3 runs at 1.17 on the same card).  Float32 MFMAs (16x16x4, 154 TFLOP/s at best) took 942 us.
+// Relative error against float64: 3.5e-7 (float32 MFMAs: 5.5e-7; they round after every 4 k, these
+// after every 32).
+//
+// MFMA operand layout (16x16x32, one wave): lane l holds A[l % 16][8g ..] and B[8g ..][l % 16] for the
+// 8 k of its lane group g = l / 16, and receives D[4g + v][l % 16], v = 0..3.
 #include <math.h>
 #include <string.h>
 
@@ -27,8 +33,19 @@
 namespace dsv {
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef float f2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bh2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bh8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+typedef f4 f4u __attribute__((aligned(4)));  // 16-byte vectors at the rows' own alignment
+typedef u4 u4u __attribute__((aligned(8)));
 
-constexpr int RS_RMAX = 512;  // R held in registers by k_rs_table (R / 4 floats a lane)
+constexpr int RS_RMAX = 512;
+constexpr int RS_B = 128;   // tile: columns of the left operand (r or h) and senders of a workgroup
+constexpr int RS_KS = 32;   // k depth of a stage: one v_mfma_f32_16x16x32_bf16
+constexpr int RS_MKS = 64;  // of a stage of the message kernel
+constexpr int RS_MPLANE = RS_B * RS_MKS * 2;
+constexpr int RS_PLANE = RS_B * RS_KS * 2;  // bytes of one bf16 part of a staged tile
 
 struct RsArgs {
   const uint16_t* raw;   // [m, H] bf16 bits (row stride raw_stride)
@@ -49,12 +66,13 @@ struct RsArgs {
   int32_t T, K, H, R, C, RR;
   int32_t n, head_is_cand;
   float eps, sqrt_c;
-  float* msg;       // [n * K, R] workspace
-  float* part;      // [slices, units, 16 + 16 * KB * 16] workspace
+  uint16_t* msg;    // [n * K, 3, R] workspace: the message's bf16 parts
+  uint16_t* wsplit; // [H, 3, R] workspace: w_last's bf16 parts
+  float* part;      // [4 slices, units, 16 + 16 * KB * 16] workspace
   float* out;       // [n, K, K]
   int32_t KB;       // ceil(K / 16): candidate blocks
   int32_t units;    // n * KB: (row, 16-sender block) pairs
-  int32_t slices, hs;  // H slices of hs columns
+  int32_t slices, hs;  // H slices of hs columns (a multiple of RS_TH)
 };
 
 __device__ __forceinline__ float bf(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
@@ -64,13 +82,51 @@ __device__ __forceinline__ f4 bf4(const uint16_t* p) {  // 4 bf16 (8-byte aligne
             __uint_as_float(w.y & 0xFFFF0000u)};
 }
 __device__ __forceinline__ f4 ld4(const float* p) { return *reinterpret_cast<const f4*>(p); }
-__device__ __forceinline__ f4 mfma4(f4 a, f4 b, f4 c) {
-  // the four k steps of a 16-wide k chunk
-  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[0], b[0], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[1], b[1], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[2], b[2], c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a[3], b[3], c, 0, 0, 0);
+__device__ __forceinline__ f4 mfma(u4 a, u4 b, f4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bh8, a), __builtin_bit_cast(bh8, b), c, 0, 0, 0);
 }
+
+// x = hi + mid + lo, each bf16 (8 significant bits, round to nearest even): exact for every finite
+// float32 above the underflow of its last bits.  An infinite x is (inf, finite, 0): its products
+// stay infinite.  Two values a call, packed.
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{a, b}), bh2));
+  const float ra = fmaxf(a - __uint_as_float(hi << 16), -1e36f);  // (inf - inf is NaN: the bound)
+  const float rb = fmaxf(b - __uint_as_float(hi & 0xFFFF0000u), -1e36f);
+  mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{ra, rb}), bh2));
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(
+                                        (f2{ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xFFFF0000u)}), bh2));
+}
+__device__ __forceinline__ void split8(const f4& x, const f4& y, u4& hi, u4& mid, u4& lo) {
+  uint32_t h, m, l;
+  split2(x[0], x[1], h, m, l);
+  hi[0] = h, mid[0] = m, lo[0] = l;
+  split2(x[2], x[3], h, m, l);
+  hi[1] = h, mid[1] = m, lo[1] = l;
+  split2(y[0], y[1], h, m, l);
+  hi[2] = h, mid[2] = m, lo[2] = l;
+  split2(y[2], y[3], h, m, l);
+  hi[3] = h, mid[3] = m, lo[3] = l;
+}
+
+// A staged tile's part: bf16 rows of 32 k, 64 bytes a row, its four 16-byte chunks (8 k each) placed
+// at chunk ^ (row / 2 % 4): eight lanes of a fragment read (eight rows, one chunk) cover the banks
+// once (placed at chunk ^ (row / 4 % 4), half of the reads' cycles were bank conflicts).
+__device__ __forceinline__ int tile_at(int row, int kc) { return row * 64 + ((kc ^ (row >> 1)) & 3) * 16; }
+// the same for stages of 64 k: 128 bytes a row, eight chunks
+__device__ __forceinline__ int tile_at64(int row, int kc) { return row * 128 + ((kc ^ (row >> 1)) & 7) * 16; }
+// 16 bytes a lane from memory to LDS (the wave's 64 chunks in lane order from `dst`)
+__device__ __forceinline__ void to_lds(const uint16_t* src, char* dst) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                   (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
+}
+// this wave's copies to LDS have landed, and every wave's; every wave is done reading the other buffer
+__device__ __forceinline__ void stage_wait() {
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+}
+__device__ __forceinline__ u4 lds16(const char* p) { return *reinterpret_cast<const u4*>(p); }
+__device__ __forceinline__ void put16(char* p, u4 v) { *reinterpret_cast<u4*>(p) = v; }
 
 // The sender token of sender row i = n * K + j: the anchor on a request's first block row, else
 // candidate j of the previous row.
@@ -85,197 +141,314 @@ __device__ __forceinline__ int64_t state_row(const RsArgs& A, int64_t n) {
 }
 
 // ---------------------------------------------------------------------------------------
-// k_rs_message: 64 sender rows x 64 R columns a workgroup (wave w: sender rows 16w..16w+15).
-// The B operands (pg and pv rows r0..r0+63) go through LDS in tiles of 64 k, shared by the four
-// waves, the next tile's loads in flight in registers while the current one is used.
+// k_rs_message: 128 sender rows x 64 R columns of both the gate and the value (the tile's 128 left
+// rows: pg rows r0.., then pv rows r0..).  Wave (w & 1, w >> 1) has 64 senders and 32 columns of
+// each; D[4g + v][li] is column 4g + v of sender li.  A stage is 64 k deep (130 us at the sizes
+// above; 32 deep, with half the products between barriers, 139 us); the weights' parts are made while
+// staging, the next stage's loads in flight in registers.
 // ---------------------------------------------------------------------------------------
-constexpr int RS_MK = 64;            // k of a staged tile (four 16-wide k steps)
-constexpr int RS_MROW = RS_MK + 4;   // LDS row stride (floats): a lane group's 16 rows of one
-                                     // k step fall in distinct bank groups
-constexpr int RS_MCH = 2 * 64 * RS_MK / 4 / 256;  // 16-byte chunks of a tile pair a thread copies
-
-__global__ __launch_bounds__(256) void k_rs_message(RsArgs A) {
-  __shared__ __align__(16) float bt[2 * 64 * RS_MROW];  // pg tile, then pv tile
+__global__ __launch_bounds__(256, 2) void k_rs_message(RsArgs A) {
+  __shared__ __align__(16) char wt[3 * RS_MPLANE];
+  __shared__ __align__(16) char et[RS_MPLANE];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, li = lane & 15;
+  const int ws = (w & 1) * 64, wr = (w >> 1) * 32;
   const int64_t Ns = (int64_t)A.n * A.K;
-  const int64_t i = (int64_t)blockIdx.x * 64 + w * 16 + li;  // the A-operand row of this lane
-  const bool live = i < Ns;
-  const int64_t sid = live ? sender_of(A, i) : 0;
+  const int64_t i0 = (int64_t)blockIdx.x * RS_B;
   const int r0 = blockIdx.y * 64;
-  const uint16_t* erow = A.codebook + sid * A.C;
-  f4 accg[4], accv[4];
+  // this thread copies chunk tid % 8 of tile rows tid / 8 + 32 c (senders; pg, then pv rows)
+  const int crow = tid >> 3, kc = tid & 7;
+  // (a row past the last sender repeats it: its column of D is dropped)
+  int64_t sid[4];
 #pragma unroll
-  for (int cb = 0; cb < 4; ++cb) accg[cb] = accv[cb] = f4{0.f, 0.f, 0.f, 0.f};
-  // tile copy: chunk q = c * 256 + tid -> matrix q / 1024, row (q % 1024) / 16, k chunk q % 16
-  f4 pre[RS_MCH];
-  auto fetch = [&](int k0) {
+  for (int c = 0; c < 4; ++c) {
+    const int64_t i = i0 + crow + 32 * c;
+    sid[c] = sender_of(A, i < Ns ? i : Ns - 1);
+  }
+  f4 acc[2][2][4];  // [gate, value][16 columns][16 senders]
 #pragma unroll
-    for (int c = 0; c < RS_MCH; ++c) {
-      const int q = c * 256 + tid, mat = q >> 10, row = (q >> 4) & 63, kc = q & 15;
-      const float* src = mat ? A.pv : A.pg;
-      if (k0 + 4 * kc < A.C) pre[c] = ld4(src + (int64_t)(r0 + row) * A.C + k0 + 4 * kc);
+  for (int i = 0; i < 16; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] = f4{0.f, 0.f, 0.f, 0.f};
+
+  // one product over `depth` (a multiple of 16): rows of `src` (bf16) times gate / value weight rows
+  auto product = [&](const uint16_t* src, const float* wg, const float* wv, int depth) {
+    u4 pe[4];
+    f4 pw[4][2];
+    auto fetch = [&](int k0) {
+      // (chunks past the depth repeat the stage's first two against zero weights)
+      const bool in = k0 + 8 * kc < depth;
+      const int k = in ? k0 + 8 * kc : k0 + 8 * (kc & 1);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        pe[c] = *reinterpret_cast<const u4u*>(src + sid[c] * depth + k);
+        const float* m = c >= 2 || !wg ? wv : wg;
+        const float* p = m + (int64_t)(r0 + crow + 32 * (c & 1)) * depth + k;
+        pw[c][0] = *reinterpret_cast<const f4u*>(p);
+        pw[c][1] = *reinterpret_cast<const f4u*>(p + 4);
+      }
+    };
+    fetch(0);
+    for (int k0 = 0; k0 < depth; k0 += RS_MKS) {
+      __syncthreads();  // (the previous stage's readers are done)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int at = tile_at64(crow + 32 * c, kc);
+        put16(et + at, pe[c]);
+        u4 hi, mid, lo;
+        split8(pw[c][0], pw[c][1], hi, mid, lo);
+        if (k0 + 8 * kc >= depth) hi = mid = lo = u4{0, 0, 0, 0};
+        put16(wt + at, hi);
+        put16(wt + RS_MPLANE + at, mid);
+        put16(wt + 2 * RS_MPLANE + at, lo);
+      }
+      __syncthreads();
+      if (k0 + RS_MKS < depth) fetch(k0 + RS_MKS);  // in flight under this stage's products
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        u4 e[4];
+#pragma unroll
+        for (int sb = 0; sb < 4; ++sb) e[sb] = lds16(et + tile_at64(ws + 16 * sb + li, 4 * ks + g));
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+          if (m == 0 && !wg) continue;
+#pragma unroll
+          for (int rb = 0; rb < 2; ++rb) {
+            const char* wp = wt + tile_at64(64 * m + wr + 16 * rb + li, 4 * ks + g);
+            const u4 hi = lds16(wp), mid = lds16(wp + RS_MPLANE), lo = lds16(wp + 2 * RS_MPLANE);
+#pragma unroll
+            for (int sb = 0; sb < 4; ++sb) acc[m][rb][sb] = mfma(lo, e[sb], acc[m][rb][sb]);
+#pragma unroll
+            for (int sb = 0; sb < 4; ++sb) acc[m][rb][sb] = mfma(mid, e[sb], acc[m][rb][sb]);
+#pragma unroll
+            for (int sb = 0; sb < 4; ++sb) acc[m][rb][sb] = mfma(hi, e[sb], acc[m][rb][sb]);
+          }
+        }
+      }
     }
   };
-  fetch(0);
-  for (int k0 = 0; k0 < A.C; k0 += RS_MK) {
-    __syncthreads();  // (the previous tile's readers are done)
+  product(A.codebook, A.pg, A.pv, A.C);
 #pragma unroll
-    for (int c = 0; c < RS_MCH; ++c) {
-      const int q = c * 256 + tid, mat = q >> 10, row = (q >> 4) & 63, kc = q & 15;
-      if (k0 + 4 * kc < A.C) *reinterpret_cast<f4*>(bt + (mat * 64 + row) * RS_MROW + 4 * kc) = pre[c];
-    }
-    __syncthreads();
-    if (k0 + RS_MK < A.C) fetch(k0 + RS_MK);  // in flight under this tile's products
-    const int ns = (A.C - k0) / 16 < RS_MK / 16 ? (A.C - k0) / 16 : RS_MK / 16;
-#pragma unroll 1
-    for (int st = 0; st < ns; ++st) {  // (ns < 4: a partial last tile when C is not a multiple of RS_MK)
-      f4 a = bf4(erow + k0 + 16 * st + 4 * g);
-      a *= A.sqrt_c;
-      if (!live) a = f4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 16; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] *= A.sqrt_c;
+  if (A.res_emb) product(A.res_emb, nullptr, A.res_proj, A.RR);  // value += res_emb[sender] @ res_proj^T
+
 #pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const float* bp = bt + (16 * cb + li) * RS_MROW + 16 * st + 4 * g;
-        accg[cb] = mfma4(a, *reinterpret_cast<const f4*>(bp), accg[cb]);
-        accv[cb] = mfma4(a, *reinterpret_cast<const f4*>(bp + 64 * RS_MROW), accv[cb]);
-      }
-    }
-  }
-  if (A.res_emb) {  // the terminal residual: value += res_emb[sender] @ res_proj^T
-    const uint16_t* rrow = A.res_emb + sid * A.RR;
-    for (int k0 = 0; k0 < A.RR; k0 += 16) {
-      f4 a = bf4(rrow + k0 + 4 * g);
-      if (!live) a = f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const int64_t r = r0 + 16 * cb + li;
-        accv[cb] = mfma4(a, ld4(A.res_proj + r * A.RR + k0 + 4 * g), accv[cb]);
-      }
-    }
-  }
-  // lane: D[4g + v][li] = sender row 16w + 4g + v, column r0 + 16cb + li
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int64_t io = (int64_t)blockIdx.x * 64 + w * 16 + 4 * g + v;
+  for (int sb = 0; sb < 4; ++sb) {
+    const int64_t io = i0 + ws + 16 * sb + li;
     if (io >= Ns) continue;
-    const int64_t mrow = state_row(A, io / A.K);
-    const uint16_t* qrow = A.query + mrow * A.query_stride;
+    const uint16_t* qrow = A.query + state_row(A, io / A.K) * A.query_stride;
 #pragma unroll
-    for (int cb = 0; cb < 4; ++cb) {
-      const int r = r0 + 16 * cb + li;
-      const float pre_ = (bf(qrow[r]) + accg[cb][v]) + A.gb[r];
-      const float gate = 1.f / (1.f + expf(-pre_));
-      A.msg[io * A.R + r] = gate * accv[cb][v];
+    for (int rb = 0; rb < 2; ++rb) {
+      const int r = r0 + wr + 16 * rb + 4 * g;
+      float msg[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float pre = (bf(qrow[r + v]) + acc[0][rb][sb][v]) + A.gb[r + v];
+        msg[v] = 1.f / (1.f + expf(-pre)) * acc[1][rb][sb][v];
+      }
+      uint2 part[3];
+      split2(msg[0], msg[1], part[0].x, part[1].x, part[2].x);
+      split2(msg[2], msg[3], part[0].y, part[1].y, part[2].y);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(A.msg + (io * 3 + q) * A.R + r) = part[q];
     }
   }
 }
 
+// w_last's bf16 parts, [H, 3, R]: eight values a thread.
+__global__ void k_rs_split(RsArgs A) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int rc = A.R / 8;
+  if (q >= (int64_t)A.H * rc) return;
+  const int64_t h = q / rc, c = q - h * rc;
+  const float* p = A.w_last + h * A.R + 8 * c;
+  u4 hi, mid, lo;
+  const f4 x = *reinterpret_cast<const f4u*>(p), y = *reinterpret_cast<const f4u*>(p + 4);
+  split8(x, y, hi, mid, lo);
+  uint16_t* o = A.wsplit + h * 3 * A.R + 8 * c;
+  *reinterpret_cast<u4*>(o) = hi;
+  *reinterpret_cast<u4*>(o + A.R) = mid;
+  *reinterpret_cast<u4*>(o + 2 * A.R) = lo;
+}
+
 // ---------------------------------------------------------------------------------------
-// k_rs_table: one (row, 16-sender block) a wave, 4 a workgroup, one H slice a grid column.  The
-// workgroup stages each 16-row tile of w_last (16 h x R) in LDS once for its four waves, the
-// next tile's loads in flight in registers while the current tile feeds the matrix cores.
+// k_rs_table: eight units (a row's 16 senders each) a workgroup, one H slice a grid column.  Wave
+// (w & 1, w >> 1) of eight has 4 units and 64 h of a 256-h tile; D[4g + v][li] is h 4g + v of
+// sender li, which two 16-h blocks at a time is the B operand of the product with the head rows.
+// A stage (32 k of the tile's w_last and message parts, 72 KB) goes from memory straight to LDS, the
+// next one into the other buffer while this one is multiplied: 300 us at the sizes above.  128-h tiles
+// of four waves with the parts of w_last made while staging through registers (two workgroups a CU)
+// took 370: the splitting, 13 spilled registers, and 1.4 times the operand traffic.
 // ---------------------------------------------------------------------------------------
-constexpr int RS_TROW = RS_RMAX + 4;  // LDS row stride of a w_last tile (floats): 16 rows' 16-byte
-                                      // A fragments of one k step fall in distinct bank groups
-constexpr int RS_TCH = 16 * RS_RMAX / 4 / 256;  // 16-byte chunks of a full tile a thread copies
+constexpr int RS_TH = 256;                    // h of a tile
+constexpr int RS_WPLANE = RS_TH * RS_KS * 2;  // bytes of one part of a stage's w_last rows
+constexpr int RS_STAGE = 3 * (RS_WPLANE + RS_PLANE);
 
 template <int KB>
-__global__ __launch_bounds__(256) void k_rs_table(RsArgs A) {
-  __shared__ __align__(16) float tile[16 * RS_TROW];
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, li = lane & 15;
-  const int unit = blockIdx.x * 4 + w;
-  const bool ulive = unit < A.units;  // (a wave past the last unit still copies tiles)
+__global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
+  __shared__ __align__(16) char buf0[RS_STAGE];
+  __shared__ __align__(16) char buf1[RS_STAGE];
+  __shared__ const uint16_t* hrows[8 * KB * 16];
+  __shared__ const uint16_t* xrows[8];
+  __shared__ float scales[8];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, li = lane & 15;
+  const int ws = (w & 1) * 64, wh = (w >> 1) * 64;
+  const int unit0 = blockIdx.x * (RS_B / 16);
   const int slice = blockIdx.y;
-  const int64_t n = ulive ? unit / KB : 0;
-  const int jb = ulive ? unit - (int)n * KB : 0;
-  const int j = jb * 16 + li;  // the sender lane of this lane's B-operand column
-  const bool jlive = ulive && j < A.K;
-  const int64_t mrow = state_row(A, n);
-  const float scale = A.rms[mrow];
-  const uint16_t* xrow = A.raw + mrow * A.raw_stride;
-  // msg of sender j in registers: lane group g holds columns 16t + 4g .. 16t + 4g + 3
-  f4 mb[RS_RMAX / 16];
-  const float* mrowp = A.msg + (n * A.K + (jlive ? j : 0)) * A.R;
-#pragma unroll
-  for (int t = 0; t < RS_RMAX / 16; ++t) {
-    mb[t] = f4{0.f, 0.f, 0.f, 0.f};
-    if (16 * t < A.R && jlive) mb[t] = ld4(mrowp + 16 * t + 4 * g);
+  // where each unit's state row and each sender column's head rows are (a unit past the last, and a
+  // lane past K, repeats one: what it computes is dropped)
+  for (int q = tid; q < 8 * KB * 16; q += 512) {
+    const int unit = unit0 + q / (KB * 16) < A.units ? unit0 + q / (KB * 16) : A.units - 1, c = q % (KB * 16);
+    const int64_t at = (int64_t)(unit / KB) * A.K + (c < A.K ? c : A.K - 1);
+    hrows[q] = A.head + (A.head_is_cand ? at : A.cand[at]) * A.H;
   }
-  // the candidates' head rows (A operand of the second product: row c = cb*16 + li)
-  const uint16_t* hrow[KB];
-  bool clive[KB];
-#pragma unroll
-  for (int cb = 0; cb < KB; ++cb) {
-    const int c = cb * 16 + li;
-    clive[cb] = ulive && c < A.K;
-    const int64_t cc = clive[cb] ? c : 0;
-    hrow[cb] = A.head_is_cand ? A.head + (n * A.K + cc) * A.H : A.head + A.cand[n * A.K + cc] * A.H;
+  if (tid < 8) {
+    const int unit = unit0 + tid < A.units ? unit0 + tid : A.units - 1;
+    const int64_t mrow = state_row(A, unit / KB);
+    xrows[tid] = A.raw + mrow * A.raw_stride;
+    scales[tid] = A.rms[mrow];
   }
-  f4 dot[KB];
-#pragma unroll
-  for (int cb = 0; cb < KB; ++cb) dot[cb] = f4{0.f, 0.f, 0.f, 0.f};
-  float ss = 0.f;
-  const int h_lo = slice * A.hs, h_hi = h_lo + A.hs;
-  // tile copy: chunk q = i * 256 + tid of the tile's 16 x R/4 chunks -> row q / (R/4), column
-  // chunk q % (R/4); chunks past 4R (R < RS_RMAX) are not copied (goff -1)
-  const int rq = A.R / 4, nq = 16 * rq;
-  int goff[RS_TCH], loff[RS_TCH];  // this thread's chunks: offsets in w_last rows h0.. and in the tile
-#pragma unroll
-  for (int i = 0; i < RS_TCH; ++i) {
-    const int q = i * 256 + tid;
-    const int row = q / rq, col = q - row * rq;
-    goff[i] = q < nq ? row * A.R + 4 * col : -1;
-    loff[i] = row * RS_TROW + 4 * col;
+  const int h_lo = slice * A.hs, h_hi = h_lo + A.hs < A.H ? h_lo + A.hs : A.H;
+  // copies: wave w fills rows 16w.. and 128 + 16w.. of each w_last part and rows 16w.. of each message
+  // part; LDS chunk (row, slot) holds the row's chunk slot ^ (row / 2 % 4) -- see tile_at
+  const int crow = 16 * w + (lane >> 2), cch = 8 * ((lane ^ (crow >> 1)) & 3);
+  const uint16_t* msrc;
+  {
+    const int unit = unit0 + w < A.units ? unit0 + w : A.units - 1, j = (unit % KB) * 16 + (lane >> 2);
+    msrc = A.msg + ((int64_t)(unit / KB) * A.K + (j < A.K ? j : A.K - 1)) * 3 * A.R + cch;
   }
-  f4 pre[RS_TCH];
-  auto fetch = [&](int h0) {
-    const float* base = A.w_last + (int64_t)h0 * A.R;
+  auto fetch = [&](char* buf, int h0, int k0) {
 #pragma unroll
-    for (int i = 0; i < RS_TCH; ++i)
-      if (goff[i] >= 0) pre[i] = ld4(base + goff[i]);
+    for (int c = 0; c < 2; ++c) {
+      const int h = h0 + 128 * c + crow < h_hi ? h0 + 128 * c + crow : h_hi - 1;
+      const uint16_t* src = A.wsplit + (int64_t)h * 3 * A.R + cch + k0;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) to_lds(src + q * A.R, buf + q * RS_WPLANE + (128 * c + 16 * w) * 64);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q) to_lds(msrc + q * A.R + k0, buf + 3 * RS_WPLANE + q * RS_PLANE + 16 * w * 64);
   };
-  fetch(h_lo);
-  for (int h0 = h_lo; h0 < h_hi; h0 += 16) {
-    __syncthreads();  // (the previous tile's readers are done)
+  f4 dot[4][KB];
+  float ss[4];
 #pragma unroll
-    for (int i = 0; i < RS_TCH; ++i)
-      if (goff[i] >= 0) *reinterpret_cast<f4*>(tile + loff[i]) = pre[i];
-    __syncthreads();
-    if (h0 + 16 < h_hi) fetch(h0 + 16);  // in flight under this tile's products
-    if (!ulive) continue;
-    // ref^T block [16 h x 16 senders]: A = w_last rows h0 + li (from the tile), B = msg^T
-    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
-    const float* arow = tile + li * RS_TROW + 4 * g;
+  for (int u = 0; u < 4; ++u) {
+    ss[u] = 0.f;
 #pragma unroll
-    for (int t = 0; t < RS_RMAX / 16; ++t)
-      if (16 * t < A.R) acc = mfma4(*reinterpret_cast<const f4*>(arow + 16 * t), mb[t], acc);
-    // lane: h = h0 + 4g + v, sender j; ref, its square, and ref * norm_w as the B operand
-    const f4 xv = bf4(xrow + h0 + 4 * g);
-    const f4 nw = ld4(A.norm_w + h0 + 4 * g);
-    f4 bv;
+    for (int cb = 0; cb < KB; ++cb) dot[u][cb] = f4{0.f, 0.f, 0.f, 0.f};
+  }
+  f4 acc[4][4];  // [16 h][unit]
+  const int wb = tile_at(wh + li, g), mb = 3 * RS_WPLANE + tile_at(ws + li, g);  // (16 rows on: 1024 bytes)
+  auto multiply = [&](const char* buf) {
+    u4 b[4][3];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float ref = xv[v] + scale * acc[v];
-      ss += ref * ref;
-      bv[v] = ref * nw[v];
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) b[u][q] = lds16(buf + mb + q * RS_PLANE + 1024 * u);
+#pragma unroll
+    for (int hb = 0; hb < 4; ++hb) {
+      const char* wp = buf + wb + 1024 * hb;
+      const u4 hi = lds16(wp), mid = lds16(wp + RS_WPLANE), lo = lds16(wp + 2 * RS_WPLANE);
+      // the products down to 2^-18 of the first, smallest first (what is left out is under 2^-25)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(lo, b[u][0], acc[hb][u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(hi, b[u][2], acc[hb][u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(mid, b[u][1], acc[hb][u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(mid, b[u][0], acc[hb][u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(hi, b[u][1], acc[hb][u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(hi, b[u][0], acc[hb][u]);
+    }
+  };
+  fetch(buf0, h_lo, 0);
+  for (int h0 = h_lo; h0 < h_hi; h0 += RS_TH) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[i >> 2][i & 3] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < A.R; k0 += 2 * RS_KS) {  // (R is a multiple of 64)
+      // (the copies are issued before the products: the compiler may not move them down)
+      stage_wait();
+      fetch(buf1, h0, k0 + RS_KS);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(buf0);
+      stage_wait();
+      const bool last = k0 + 2 * RS_KS >= A.R;
+      const int nh = last ? h0 + RS_TH : h0;
+      if (nh < h_hi) fetch(buf0, nh, last ? 0 : k0 + 2 * RS_KS);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(buf1);
+    }
+    // ref, its square, and (ref * norm_w) . head.  A 16-h block past the slice repeats its last one
+    // (H is a multiple of 16) with ref 0; its operands are loaded four units at a time, before use
+    const bool whole = h0 + wh + 64 <= h_hi;
+    int hx[4];
+    f4 nw[4];
+#pragma unroll
+    for (int hb = 0; hb < 4; ++hb) {
+      const int h = h0 + wh + 16 * hb;
+      hx[hb] = (h < h_hi ? h : h_hi - 16) + 4 * g;
+      nw[hb] = *reinterpret_cast<const f4u*>(A.norm_w + hx[hb]);
+    }
+    uint2 xb[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const uint16_t* xrow = xrows[(ws >> 4) + u];
+#pragma unroll
+      for (int hb = 0; hb < 4; ++hb) xb[u][hb] = *reinterpret_cast<const uint2*>(xrow + hx[hb]);
     }
 #pragma unroll
     for (int cb = 0; cb < KB; ++cb) {
-      f4 a = bf4(hrow[cb] + h0 + 4 * g);
-      if (!clive[cb]) a = f4{0.f, 0.f, 0.f, 0.f};
-      dot[cb] = mfma4(a, bv, dot[cb]);
+      uint2 hd[4][4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint16_t* hrow = hrows[((ws >> 4) + u) * KB * 16 + cb * 16 + li];
+#pragma unroll
+        for (int hb = 0; hb < 4; ++hb) hd[u][hb] = *reinterpret_cast<const uint2*>(hrow + hx[hb]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (cb == 0) {
+          const float scale = scales[(ws >> 4) + u];
+#pragma unroll
+          for (int hb = 0; hb < 4; ++hb) {
+            const bool in = whole || h0 + wh + 16 * hb < h_hi;
+            const f4 xv = {__uint_as_float(xb[u][hb].x << 16), __uint_as_float(xb[u][hb].x & 0xFFFF0000u),
+                           __uint_as_float(xb[u][hb].y << 16), __uint_as_float(xb[u][hb].y & 0xFFFF0000u)};
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              const float ref = in ? xv[v] + scale * acc[hb][u][v] : 0.f;
+              ss[u] += ref * ref;
+              acc[hb][u][v] = ref * nw[hb][v];
+            }
+          }
+        }
+#pragma unroll
+        for (int hp = 0; hp < 4; hp += 2) {
+          u4 hi, mid, lo;
+          split8(acc[hp][u], acc[hp + 1][u], hi, mid, lo);
+          const u4 a = {hd[u][hp].x, hd[u][hp].y, hd[u][hp + 1].x, hd[u][hp + 1].y};
+          dot[u][cb] = mfma(a, lo, dot[u][cb]);
+          dot[u][cb] = mfma(a, mid, dot[u][cb]);
+          dot[u][cb] = mfma(a, hi, dot[u][cb]);
+        }
+      }
     }
   }
-  if (!ulive) return;
-  // the slice's partial sums: ss over the lane group's h (lanes li, li+16, li+32, li+48 share j),
-  // dot[cb][v] = sum_h head[c = cb*16 + 4g + v][h] * ref[j][h] * norm_w[h]
-  ss += __shfl_xor(ss, 16);
-  ss += __shfl_xor(ss, 32);
-  float* pp = A.part + ((int64_t)slice * A.units + unit) * (16 + 16 * KB * 16);
-  if (g == 0) pp[li] = ss;
+  // the wave's partial sums: ss over the lane groups' h (lanes li, li+16, li+32, li+48 share a sender),
+  // dot[u][cb][v] = sum_h head[c = cb*16 + 4g + v][h] * ref[j][h] * norm_w[h]
 #pragma unroll
-  for (int cb = 0; cb < KB; ++cb)
+  for (int u = 0; u < 4; ++u) {
+    const int unit = unit0 + (ws >> 4) + u;
+    if (unit >= A.units) continue;
+    float s = ss[u];
+    s += __shfl_xor(s, 16);
+    s += __shfl_xor(s, 32);
+    float* pp = A.part + ((int64_t)(slice * 4 + (w >> 1)) * A.units + unit) * (16 + 16 * KB * 16);
+    if (g == 0) pp[li] = s;
 #pragma unroll
-    for (int v = 0; v < 4; ++v) pp[16 + (cb * 16 + 4 * g + v) * 16 + li] = dot[cb][v];
+    for (int cb = 0; cb < KB; ++cb)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) pp[16 + (cb * 16 + 4 * g + v) * 16 + li] = dot[u][cb][v];
+  }
 }
 
 // out[n, j, c] = (sum over slices of the dot products) / sqrt(sum of ref^2 / H + eps)
@@ -288,7 +461,7 @@ __global__ void k_rs_finish(RsArgs A) {
   const int unit = (int)n * A.KB + j / 16, jl = j % 16;
   const int stride = 16 + 16 * A.KB * 16;
   float ss = 0.f, d = 0.f;
-  for (int s = 0; s < A.slices; ++s) {
+  for (int s = 0; s < 4 * A.slices; ++s) {
     const float* pp = A.part + ((int64_t)s * A.units + unit) * stride;
     ss += pp[jl];
     d += pp[16 + c * 16 + jl];
@@ -300,10 +473,21 @@ __global__ void k_rs_finish(RsArgs A) {
 
 using namespace dsv;
 
+// H slices of a call: a workgroup a CU, a tile of RS_TH h each at least.
+static int rs_slices(int64_t units, int32_t H) {
+  const int64_t blocks = (units + RS_B / 16 - 1) / (RS_B / 16), tiles = (H + RS_TH - 1) / RS_TH;
+  const int64_t want = blocks >= 256 ? 1 : 256 / blocks;
+  return (int)(want < tiles ? want : tiles);
+}
+static int64_t rs_round(int64_t bytes) { return (bytes + 255) / 256 * 256; }
+
+// (a bound that grows with n: a workspace sized for n serves every smaller n.  units * slices is at
+// most units * tiles, and at most 8 * 256 while there is more than one slice)
 extern "C" int64_t dsv_rs_table_workspace_bytes(int64_t n, int32_t K, int32_t H, int32_t R) {
-  const int64_t KB = (K + 15) / 16;
-  const int64_t slices = H % 128 == 0 ? 8 : 1;
-  return n * K * R * 4 + slices * n * KB * (16 + 16 * KB * 16) * 4 + 256;
+  const int64_t KB = (K + 15) / 16, units = n * KB, tiles = (H + RS_TH - 1) / RS_TH;
+  int64_t us = units * tiles < 2048 ? units * tiles : 2048;
+  if (us < units) us = units;
+  return rs_round(n * K * R * 6) + rs_round((int64_t)H * R * 6) + 4 * us * (16 + 16 * KB * 16) * 4 + 256;
 }
 
 extern "C" int dsv_rs_table(const void* raw, int64_t raw_stride, const float* rms, const void* query,
@@ -359,21 +543,24 @@ extern "C" int dsv_rs_table(const void* raw, int64_t raw_stride, const float* rm
   A.sqrt_c = (float)sqrt((double)C);
   A.KB = (K + 15) / 16;
   A.units = (int32_t)n * A.KB;
-  A.slices = H % 128 == 0 ? 8 : 1;
-  A.hs = H / A.slices;
-  char* ws = reinterpret_cast<char*>(workspace);
-  A.msg = reinterpret_cast<float*>(ws);
-  A.part = reinterpret_cast<float*>(ws + (((int64_t)n * K * R * 4 + 255) / 256) * 256);
+  A.slices = rs_slices(A.units, H);
+  A.hs = ((H + RS_TH - 1) / RS_TH + A.slices - 1) / A.slices * RS_TH;
+  A.slices = (H + A.hs - 1) / A.hs;  // (none of them empty)
+  char* ws = reinterpret_cast<char*>(rs_round((int64_t)workspace));  // (16-byte copies; the size has 256 spare)
+  A.msg = reinterpret_cast<uint16_t*>(ws);
+  A.wsplit = reinterpret_cast<uint16_t*>(ws + rs_round(n * K * R * 6));
+  A.part = reinterpret_cast<float*>(ws + rs_round(n * K * R * 6) + rs_round((int64_t)H * R * 6));
   A.out = out;
   const int64_t Ns = n * K;
-  hipLaunchKernelGGL(k_rs_message, dim3((unsigned)((Ns + 63) / 64), (unsigned)(R / 64)), dim3(256), 0, stream, A);
-  DSV_CHECK_LAUNCH("k_rs_message");
-  const dim3 tg((unsigned)((A.units + 3) / 4), (unsigned)A.slices);
+  hipLaunchKernelGGL(k_rs_message, dim3((unsigned)((Ns + RS_B - 1) / RS_B), (unsigned)(R / 64)), dim3(256), 0, stream, A);
+  hipLaunchKernelGGL(k_rs_split, dim3((unsigned)(((int64_t)H * R / 8 + 255) / 256)), dim3(256), 0, stream, A);
+  DSV_CHECK_LAUNCH("k_rs_message / k_rs_split");
+  const dim3 tg((unsigned)((A.units + RS_B / 16 - 1) / (RS_B / 16)), (unsigned)A.slices);
   switch (A.KB) {
-    case 1: hipLaunchKernelGGL(k_rs_table<1>, tg, dim3(256), 0, stream, A); break;
-    case 2: hipLaunchKernelGGL(k_rs_table<2>, tg, dim3(256), 0, stream, A); break;
-    case 3: hipLaunchKernelGGL(k_rs_table<3>, tg, dim3(256), 0, stream, A); break;
-    default: hipLaunchKernelGGL(k_rs_table<4>, tg, dim3(256), 0, stream, A); break;
+    case 1: hipLaunchKernelGGL(k_rs_table<1>, tg, dim3(512), 0, stream, A); break;
+    case 2: hipLaunchKernelGGL(k_rs_table<2>, tg, dim3(512), 0, stream, A); break;
+    case 3: hipLaunchKernelGGL(k_rs_table<3>, tg, dim3(512), 0, stream, A); break;
+    default: hipLaunchKernelGGL(k_rs_table<4>, tg, dim3(512), 0, stream, A); break;
   }
   DSV_CHECK_LAUNCH("k_rs_table");
   const int64_t total = n * K * K;

@@ -378,7 +378,8 @@ int dsv_sps_plan(const float* raw, int64_t raw_stride, int32_t bs, int32_t gamma
                  int32_t* qo_indptr, int64_t* window_index, dsv_stream_t stream);
 
 /* Draft-side sampling table of the serial last-write refinement (kernels/dspine.py:505-613,  */
-/* serial_rs_table), float32 on the matrix cores: out [n, K, K] with n = bs * (T - 1) block    */
+/* serial_rs_table), float32 accuracy on the matrix cores (three bf16 parts a float32 operand): */
+/* out [n, K, K] with n = bs * (T - 1) block                                                   */
 /* rows, out[n, j, c] = normalize(raw[r] + rms[r] * ((sigmoid(query[r] + e_j pg^T + gb) *     */
 /* (e_j pv^T + res_j res_proj^T)) write_w^T)) * norm_w . head[n, c], r = the row's state row,  */
 /* e_j = sqrt(C) * codebook[sender j] (the anchor on a request's first block row, else        */

@@ -82,6 +82,38 @@ def test_table_candidate_widths(device, k):
     torch.testing.assert_close(table.double(), _ref(d, T), rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("bs,T,H,R,C,k,scale", [
+    (1, 2, 16, 64, 16, 1, 1.0),       # one sender, one 16-h block, half a stage of C
+    (3, 4, 272, 320, 80, 17, 1.0),    # two lane blocks, a unit block and an H tile that end early, C % 64 = 16
+    (5, 6, 1040, 128, 144, 24, 1e18),  # weights far from 1: the parts keep float32's exponents
+    (13, 2, 528, 512, 272, 9, 1e-18),
+    (2, 9, 256, 192, 64, 48, 1.0),    # three lane blocks
+])
+def test_table_tile_edges(device, bs, T, H, R, C, k, scale):
+    """Sizes that end inside the kernels' tiles (128 senders, 256 h, 64 k), in the 2-norm: float32
+    sums of C, R and H terms round to about 2^-24 (sqrt(C) + sqrt(R) + sqrt(H)) of their size."""
+    d = _inputs(31, bs=bs, T=T, H=H, R=R, C=C, V=512, k=k)
+    d["w_last"] = d["w_last"] * scale
+    d["rms"] = d["rms"] / scale
+    table = _gpu_table(d, T, device).cpu().double()
+    ref = _ref(d, T)
+    bound = 2.0 ** -24 * (math.sqrt(C) + math.sqrt(R) + math.sqrt(H))
+    assert float((table - ref).norm() / ref.norm()) < bound
+    assert torch.isfinite(table).all()
+
+
+def test_table_infinite_weight_saturates_the_gate(device):
+    """A gate weight of -inf against a positive code closes that column's gate (sigmoid(-inf) = 0) and
+    leaves the rest finite; of +inf opens it."""
+    T = 3
+    d = _inputs(8, bs=2, T=T, H=64, R=64, C=16, V=64, k=4)
+    d["codebook"] = d["codebook"].abs() + 0.125
+    d["pg"][3, :], d["pg"][7, 5] = -math.inf, math.inf
+    table = _gpu_table(d, T, device).cpu()
+    assert torch.isfinite(table).all()
+    torch.testing.assert_close(table.double(), _ref(d, T), rtol=1e-4, atol=1e-4)
+
+
 def test_table_residual_and_candidate_head(device):
     """The terminal residual added to the value, and head rows given per candidate
     ([n, K, H] instead of lm_head gathered by id)."""
