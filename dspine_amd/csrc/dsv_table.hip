@@ -7,10 +7,10 @@
 //   T[n, j, c] = (ref / sqrt(mean(ref^2) + eps) * norm_w) . head[n, c]
 // in float32 accuracy on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16, float32 accumulation): a
 // float32 operand is three bf16 parts (split2), a bf16 operand one, and a product of two float32
-// operands is the six part products that reach float32's last bit.  Four launches:
+// operands is the six part products that reach float32's last bit.  Three launches:
 //   k_rs_message  sender rows x R: the gathered codebook rows times [pg; pv]^T, scaled, with the gate,
-//                 the value and their product in the epilogue -> msg's parts [n*K, 3, R]
-//   k_rs_split    w_last's parts [H, 3, R]
+//                 the value and their product in the epilogue -> msg's parts [n*K, 3, R]; its last
+//                 workgroups make w_last's parts [H, 3, R]
 //   k_rs_table    (eight units of 16 senders, H slice): msg times w_last^T in 16 x 16 output blocks
 //                 that are already the B operand of the second product against the 16 candidates'
 //                 head rows, so ref never leaves registers; partial sums of ref^2 and of the dot
@@ -44,7 +44,6 @@ constexpr int RS_RMAX = 512;
 constexpr int RS_B = 128;   // tile: columns of the left operand (r or h) and senders of a workgroup
 constexpr int RS_KS = 32;   // k depth of a stage: one v_mfma_f32_16x16x32_bf16
 constexpr int RS_MKS = 64;  // of a stage of the message kernel
-constexpr int RS_MPLANE = RS_B * RS_MKS * 2;
 constexpr int RS_PLANE = RS_B * RS_KS * 2;  // bytes of one bf16 part of a staged tile
 
 struct RsArgs {
@@ -68,11 +67,12 @@ struct RsArgs {
   float eps, sqrt_c;
   uint16_t* msg;    // [n * K, 3, R] workspace: the message's bf16 parts
   uint16_t* wsplit; // [H, 3, R] workspace: w_last's bf16 parts
-  float* part;      // [4 slices, units, 16 + 16 * KB * 16] workspace
+  float* part;      // [parts, units, 16 + 16 * KB * 16] workspace
   float* out;       // [n, K, K]
   int32_t KB;       // ceil(K / 16): candidate blocks
   int32_t units;    // n * KB: (row, 16-sender block) pairs
-  int32_t slices, hs;  // H slices of hs columns (a multiple of RS_TH)
+  int32_t hs, parts;  // columns of an H slice (a multiple of the tile's); partial sums a unit leaves
+  int32_t sblocks;  // 128-sender blocks of the message
 };
 
 __device__ __forceinline__ float bf(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
@@ -147,14 +147,37 @@ __device__ __forceinline__ int64_t state_row(const RsArgs& A, int64_t n) {
 // above; 32 deep, with half the products between barriers, 139 us); the weights' parts are made while
 // staging, the next stage's loads in flight in registers.
 // ---------------------------------------------------------------------------------------
+// w_last's parts, [H, 3, R]: eight values a thread.
+__device__ __forceinline__ void split_w_last(const RsArgs& A, int64_t q) {
+  const int rc = A.R / 8;
+  if (q >= (int64_t)A.H * rc) return;
+  const int64_t h = q / rc, c = q - h * rc;
+  const float* p = A.w_last + h * A.R + 8 * c;
+  u4 hi, mid, lo;
+  const f4 x = *reinterpret_cast<const f4u*>(p), y = *reinterpret_cast<const f4u*>(p + 4);
+  split8(x, y, hi, mid, lo);
+  uint16_t* o = A.wsplit + h * 3 * A.R + 8 * c;
+  *reinterpret_cast<u4*>(o) = hi;
+  *reinterpret_cast<u4*>(o + A.R) = mid;
+  *reinterpret_cast<u4*>(o + 2 * A.R) = lo;
+}
+
+template <int RC>
 __global__ __launch_bounds__(256, 2) void k_rs_message(RsArgs A) {
-  __shared__ __align__(16) char wt[3 * RS_MPLANE];
-  __shared__ __align__(16) char et[RS_MPLANE];
+  constexpr int NS = RC == 64 ? 4 : 2, NR = RC == 64 ? 2 : 1;  // a wave's 16-sender and 16-column blocks
+  constexpr int NW = RC / 16, PLANE = 2 * RC * RS_MKS * 2;     // weight chunks a thread copies; bytes of a part
+  __shared__ __align__(16) char wt[3 * PLANE];
+  __shared__ __align__(16) char et[RS_B * RS_MKS * 2];
+  const int mblocks = A.sblocks * (A.R / RC);
+  if ((int)blockIdx.x >= mblocks) {
+    split_w_last(A, (int64_t)(blockIdx.x - mblocks) * 256 + threadIdx.x);
+    return;
+  }
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, li = lane & 15;
-  const int ws = (w & 1) * 64, wr = (w >> 1) * 32;
+  const int ws = RC == 64 ? (w & 1) * 64 : w * 32, wr = RC == 64 ? (w >> 1) * 32 : 0;
   const int64_t Ns = (int64_t)A.n * A.K;
-  const int64_t i0 = (int64_t)blockIdx.x * RS_B;
-  const int r0 = blockIdx.y * 64;
+  const int64_t i0 = (int64_t)(blockIdx.x % A.sblocks) * RS_B;
+  const int r0 = (int)(blockIdx.x / A.sblocks) * RC;
   // this thread copies chunk tid % 8 of tile rows tid / 8 + 32 c (senders; pg, then pv rows)
   const int crow = tid >> 3, kc = tid & 7;
   // (a row past the last sender repeats it: its column of D is dropped)
@@ -164,23 +187,25 @@ __global__ __launch_bounds__(256, 2) void k_rs_message(RsArgs A) {
     const int64_t i = i0 + crow + 32 * c;
     sid[c] = sender_of(A, i < Ns ? i : Ns - 1);
   }
-  f4 acc[2][2][4];  // [gate, value][16 columns][16 senders]
+  f4 acc[2][NR][NS];  // [gate, value][16 columns][16 senders]
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] = f4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < 2 * NR * NS; ++i) acc[i / (NR * NS)][i / NS % NR][i % NS] = f4{0.f, 0.f, 0.f, 0.f};
 
   // one product over `depth` (a multiple of 16): rows of `src` (bf16) times gate / value weight rows
   auto product = [&](const uint16_t* src, const float* wg, const float* wv, int depth) {
     u4 pe[4];
-    f4 pw[4][2];
+    f4 pw[NW][2];
     auto fetch = [&](int k0) {
       // (chunks past the depth repeat the stage's first two against zero weights)
       const bool in = k0 + 8 * kc < depth;
       const int k = in ? k0 + 8 * kc : k0 + 8 * (kc & 1);
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        pe[c] = *reinterpret_cast<const u4u*>(src + sid[c] * depth + k);
-        const float* m = c >= 2 || !wg ? wv : wg;
-        const float* p = m + (int64_t)(r0 + crow + 32 * (c & 1)) * depth + k;
+      for (int c = 0; c < 4; ++c) pe[c] = *reinterpret_cast<const u4u*>(src + sid[c] * depth + k);
+#pragma unroll
+      for (int c = 0; c < NW; ++c) {
+        const int row = crow + 32 * c;  // (of gate rows, then value rows)
+        const float* m = row >= RC || !wg ? wv : wg;
+        const float* p = m + (int64_t)(r0 + row % RC) * depth + k;
         pw[c][0] = *reinterpret_cast<const f4u*>(p);
         pw[c][1] = *reinterpret_cast<const f4u*>(p + 4);
       }
@@ -189,36 +214,37 @@ __global__ __launch_bounds__(256, 2) void k_rs_message(RsArgs A) {
     for (int k0 = 0; k0 < depth; k0 += RS_MKS) {
       __syncthreads();  // (the previous stage's readers are done)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int at = tile_at64(crow + 32 * c, kc);
-        put16(et + at, pe[c]);
+      for (int c = 0; c < 4; ++c) put16(et + tile_at64(crow + 32 * c, kc), pe[c]);
+#pragma unroll
+      for (int c = 0; c < NW; ++c) {
         u4 hi, mid, lo;
         split8(pw[c][0], pw[c][1], hi, mid, lo);
         if (k0 + 8 * kc >= depth) hi = mid = lo = u4{0, 0, 0, 0};
-        put16(wt + at, hi);
-        put16(wt + RS_MPLANE + at, mid);
-        put16(wt + 2 * RS_MPLANE + at, lo);
+        char* at = wt + tile_at64(crow + 32 * c, kc);
+        put16(at, hi);
+        put16(at + PLANE, mid);
+        put16(at + 2 * PLANE, lo);
       }
       __syncthreads();
       if (k0 + RS_MKS < depth) fetch(k0 + RS_MKS);  // in flight under this stage's products
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        u4 e[4];
+        u4 e[NS];
 #pragma unroll
-        for (int sb = 0; sb < 4; ++sb) e[sb] = lds16(et + tile_at64(ws + 16 * sb + li, 4 * ks + g));
+        for (int sb = 0; sb < NS; ++sb) e[sb] = lds16(et + tile_at64(ws + 16 * sb + li, 4 * ks + g));
 #pragma unroll
         for (int m = 0; m < 2; ++m) {
           if (m == 0 && !wg) continue;
 #pragma unroll
-          for (int rb = 0; rb < 2; ++rb) {
-            const char* wp = wt + tile_at64(64 * m + wr + 16 * rb + li, 4 * ks + g);
-            const u4 hi = lds16(wp), mid = lds16(wp + RS_MPLANE), lo = lds16(wp + 2 * RS_MPLANE);
+          for (int rb = 0; rb < NR; ++rb) {
+            const char* wp = wt + tile_at64(RC * m + wr + 16 * rb + li, 4 * ks + g);
+            const u4 hi = lds16(wp), mid = lds16(wp + PLANE), lo = lds16(wp + 2 * PLANE);
 #pragma unroll
-            for (int sb = 0; sb < 4; ++sb) acc[m][rb][sb] = mfma(lo, e[sb], acc[m][rb][sb]);
+            for (int sb = 0; sb < NS; ++sb) acc[m][rb][sb] = mfma(lo, e[sb], acc[m][rb][sb]);
 #pragma unroll
-            for (int sb = 0; sb < 4; ++sb) acc[m][rb][sb] = mfma(mid, e[sb], acc[m][rb][sb]);
+            for (int sb = 0; sb < NS; ++sb) acc[m][rb][sb] = mfma(mid, e[sb], acc[m][rb][sb]);
 #pragma unroll
-            for (int sb = 0; sb < 4; ++sb) acc[m][rb][sb] = mfma(hi, e[sb], acc[m][rb][sb]);
+            for (int sb = 0; sb < NS; ++sb) acc[m][rb][sb] = mfma(hi, e[sb], acc[m][rb][sb]);
           }
         }
       }
@@ -226,16 +252,16 @@ __global__ __launch_bounds__(256, 2) void k_rs_message(RsArgs A) {
   };
   product(A.codebook, A.pg, A.pv, A.C);
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i >> 3][(i >> 2) & 1][i & 3] *= A.sqrt_c;
+  for (int i = 0; i < 2 * NR * NS; ++i) acc[i / (NR * NS)][i / NS % NR][i % NS] *= A.sqrt_c;
   if (A.res_emb) product(A.res_emb, nullptr, A.res_proj, A.RR);  // value += res_emb[sender] @ res_proj^T
 
 #pragma unroll
-  for (int sb = 0; sb < 4; ++sb) {
+  for (int sb = 0; sb < NS; ++sb) {
     const int64_t io = i0 + ws + 16 * sb + li;
     if (io >= Ns) continue;
     const uint16_t* qrow = A.query + state_row(A, io / A.K) * A.query_stride;
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < NR; ++rb) {
       const int r = r0 + wr + 16 * rb + 4 * g;
       float msg[4];
 #pragma unroll
@@ -252,39 +278,22 @@ __global__ __launch_bounds__(256, 2) void k_rs_message(RsArgs A) {
   }
 }
 
-// w_last's bf16 parts, [H, 3, R]: eight values a thread.
-__global__ void k_rs_split(RsArgs A) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int rc = A.R / 8;
-  if (q >= (int64_t)A.H * rc) return;
-  const int64_t h = q / rc, c = q - h * rc;
-  const float* p = A.w_last + h * A.R + 8 * c;
-  u4 hi, mid, lo;
-  const f4 x = *reinterpret_cast<const f4u*>(p), y = *reinterpret_cast<const f4u*>(p + 4);
-  split8(x, y, hi, mid, lo);
-  uint16_t* o = A.wsplit + h * 3 * A.R + 8 * c;
-  *reinterpret_cast<u4*>(o) = hi;
-  *reinterpret_cast<u4*>(o + A.R) = mid;
-  *reinterpret_cast<u4*>(o + 2 * A.R) = lo;
-}
-
 // ---------------------------------------------------------------------------------------
 // k_rs_table: eight units (a row's 16 senders each) a workgroup, one H slice a grid column.  Wave
-// (w & 1, w >> 1) of eight has 4 units and 64 h of a 256-h tile; D[4g + v][li] is h 4g + v of
+// (w & 1, w >> 1) has 4 units and 64 h of a TH-h tile (256 or 64: rs_plan); D[4g + v][li] is h 4g + v of
 // sender li, which two 16-h blocks at a time is the B operand of the product with the head rows.
 // A stage (32 k of the tile's w_last and message parts, 72 KB) goes from memory straight to LDS, the
 // next one into the other buffer while this one is multiplied: 300 us at the sizes above.  128-h tiles
 // of four waves with the parts of w_last made while staging through registers (two workgroups a CU)
 // took 370: the splitting, 13 spilled registers, and 1.4 times the operand traffic.
 // ---------------------------------------------------------------------------------------
-constexpr int RS_TH = 256;                    // h of a tile
-constexpr int RS_WPLANE = RS_TH * RS_KS * 2;  // bytes of one part of a stage's w_last rows
-constexpr int RS_STAGE = 3 * (RS_WPLANE + RS_PLANE);
-
-template <int KB>
-__global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
-  __shared__ __align__(16) char buf0[RS_STAGE];
-  __shared__ __align__(16) char buf1[RS_STAGE];
+template <int KB, int TH>
+__global__ __launch_bounds__(2 * TH, TH == 256 && KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
+  constexpr int NWAVE = TH / 32;           // waves: two of 64 senders each for every 64 h
+  constexpr int WPLANE = TH * RS_KS * 2;   // bytes of one part of a stage's w_last rows
+  constexpr int STAGE = 3 * (WPLANE + RS_PLANE);
+  __shared__ __align__(16) char buf0[STAGE];
+  __shared__ __align__(16) char buf1[STAGE];
   __shared__ const uint16_t* hrows[8 * KB * 16];
   __shared__ const uint16_t* xrows[8];
   __shared__ float scales[8];
@@ -292,9 +301,35 @@ __global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
   const int ws = (w & 1) * 64, wh = (w >> 1) * 64;
   const int unit0 = blockIdx.x * (RS_B / 16);
   const int slice = blockIdx.y;
+  const int h_lo = slice * A.hs, h_hi = h_lo + A.hs < A.H ? h_lo + A.hs : A.H;
+  // copies: 16 rows of 64 bytes a wave at a time, w_last's parts (rows 16 (w + NWAVE c)) and then the
+  // messages'; LDS chunk (row, slot) holds the row's chunk slot ^ (row / 2 % 4) -- see tile_at
+  constexpr int NC = TH / 16 / NWAVE, NM = RS_B / 16 / NWAVE;  // row blocks of each a wave copies
+  const int cch = 8 * ((lane ^ (lane >> 3)) & 3);
+  const uint16_t* msrc[NM];
+#pragma unroll
+  for (int c = 0; c < NM; ++c) {
+    const int u = unit0 + w + NWAVE * c, unit = u < A.units ? u : A.units - 1, j = (unit % KB) * 16 + (lane >> 2);
+    msrc[c] = A.msg + ((int64_t)(unit / KB) * A.K + (j < A.K ? j : A.K - 1)) * 3 * A.R + cch;
+  }
+  auto fetch = [&](char* buf, int h0, int k0) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int row = 16 * (w + NWAVE * c), h = h0 + row + (lane >> 2);
+      const uint16_t* src = A.wsplit + (int64_t)(h < h_hi ? h : h_hi - 1) * 3 * A.R + cch + k0;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) to_lds(src + q * A.R, buf + q * WPLANE + row * 64);
+    }
+#pragma unroll
+    for (int c = 0; c < NM; ++c)
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        to_lds(msrc[c] + q * A.R + k0, buf + 3 * WPLANE + q * RS_PLANE + 16 * (w + NWAVE * c) * 64);
+  };
+  fetch(buf0, h_lo, 0);
   // where each unit's state row and each sender column's head rows are (a unit past the last, and a
   // lane past K, repeats one: what it computes is dropped)
-  for (int q = tid; q < 8 * KB * 16; q += 512) {
+  for (int q = tid; q < 8 * KB * 16; q += 64 * NWAVE) {
     const int unit = unit0 + q / (KB * 16) < A.units ? unit0 + q / (KB * 16) : A.units - 1, c = q % (KB * 16);
     const int64_t at = (int64_t)(unit / KB) * A.K + (c < A.K ? c : A.K - 1);
     hrows[q] = A.head + (A.head_is_cand ? at : A.cand[at]) * A.H;
@@ -305,26 +340,6 @@ __global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
     xrows[tid] = A.raw + mrow * A.raw_stride;
     scales[tid] = A.rms[mrow];
   }
-  const int h_lo = slice * A.hs, h_hi = h_lo + A.hs < A.H ? h_lo + A.hs : A.H;
-  // copies: wave w fills rows 16w.. and 128 + 16w.. of each w_last part and rows 16w.. of each message
-  // part; LDS chunk (row, slot) holds the row's chunk slot ^ (row / 2 % 4) -- see tile_at
-  const int crow = 16 * w + (lane >> 2), cch = 8 * ((lane ^ (crow >> 1)) & 3);
-  const uint16_t* msrc;
-  {
-    const int unit = unit0 + w < A.units ? unit0 + w : A.units - 1, j = (unit % KB) * 16 + (lane >> 2);
-    msrc = A.msg + ((int64_t)(unit / KB) * A.K + (j < A.K ? j : A.K - 1)) * 3 * A.R + cch;
-  }
-  auto fetch = [&](char* buf, int h0, int k0) {
-#pragma unroll
-    for (int c = 0; c < 2; ++c) {
-      const int h = h0 + 128 * c + crow < h_hi ? h0 + 128 * c + crow : h_hi - 1;
-      const uint16_t* src = A.wsplit + (int64_t)h * 3 * A.R + cch + k0;
-#pragma unroll
-      for (int q = 0; q < 3; ++q) to_lds(src + q * A.R, buf + q * RS_WPLANE + (128 * c + 16 * w) * 64);
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) to_lds(msrc + q * A.R + k0, buf + 3 * RS_WPLANE + q * RS_PLANE + 16 * w * 64);
-  };
   f4 dot[4][KB];
   float ss[4];
 #pragma unroll
@@ -334,7 +349,7 @@ __global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
     for (int cb = 0; cb < KB; ++cb) dot[u][cb] = f4{0.f, 0.f, 0.f, 0.f};
   }
   f4 acc[4][4];  // [16 h][unit]
-  const int wb = tile_at(wh + li, g), mb = 3 * RS_WPLANE + tile_at(ws + li, g);  // (16 rows on: 1024 bytes)
+  const int wb = tile_at(wh + li, g), mb = 3 * WPLANE + tile_at(ws + li, g);  // (16 rows on: 1024 bytes)
   auto multiply = [&](const char* buf) {
     u4 b[4][3];
 #pragma unroll
@@ -344,7 +359,7 @@ __global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
 #pragma unroll
     for (int hb = 0; hb < 4; ++hb) {
       const char* wp = buf + wb + 1024 * hb;
-      const u4 hi = lds16(wp), mid = lds16(wp + RS_WPLANE), lo = lds16(wp + 2 * RS_WPLANE);
+      const u4 hi = lds16(wp), mid = lds16(wp + WPLANE), lo = lds16(wp + 2 * WPLANE);
       // the products down to 2^-18 of the first, smallest first (what is left out is under 2^-25)
 #pragma unroll
       for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(lo, b[u][0], acc[hb][u]);
@@ -360,8 +375,7 @@ __global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
       for (int u = 0; u < 4; ++u) acc[hb][u] = mfma(hi, b[u][0], acc[hb][u]);
     }
   };
-  fetch(buf0, h_lo, 0);
-  for (int h0 = h_lo; h0 < h_hi; h0 += RS_TH) {
+  for (int h0 = h_lo; h0 < h_hi; h0 += TH) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i >> 2][i & 3] = f4{0.f, 0.f, 0.f, 0.f};
     for (int k0 = 0; k0 < A.R; k0 += 2 * RS_KS) {  // (R is a multiple of 64)
@@ -372,7 +386,7 @@ __global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
       multiply(buf0);
       stage_wait();
       const bool last = k0 + 2 * RS_KS >= A.R;
-      const int nh = last ? h0 + RS_TH : h0;
+      const int nh = last ? h0 + TH : h0;
       if (nh < h_hi) fetch(buf0, nh, last ? 0 : k0 + 2 * RS_KS);
       __builtin_amdgcn_sched_barrier(0);
       multiply(buf1);
@@ -442,7 +456,7 @@ __global__ __launch_bounds__(512, KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
     float s = ss[u];
     s += __shfl_xor(s, 16);
     s += __shfl_xor(s, 32);
-    float* pp = A.part + ((int64_t)(slice * 4 + (w >> 1)) * A.units + unit) * (16 + 16 * KB * 16);
+    float* pp = A.part + ((int64_t)(slice * (TH / 64) + (w >> 1)) * A.units + unit) * (16 + 16 * KB * 16);
     if (g == 0) pp[li] = s;
 #pragma unroll
     for (int cb = 0; cb < KB; ++cb)
@@ -461,10 +475,19 @@ __global__ void k_rs_finish(RsArgs A) {
   const int unit = (int)n * A.KB + j / 16, jl = j % 16;
   const int stride = 16 + 16 * A.KB * 16;
   float ss = 0.f, d = 0.f;
-  for (int s = 0; s < 4 * A.slices; ++s) {
-    const float* pp = A.part + ((int64_t)s * A.units + unit) * stride;
-    ss += pp[jl];
-    d += pp[16 + c * 16 + jl];
+  const float* pp = A.part + (int64_t)unit * stride;
+  const int64_t step = (int64_t)A.units * stride;
+  for (int s = 0; s < A.parts; s += 8) {  // eight parts' loads in flight (one by one: 24 us for 64 parts)
+    float a[8], b[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const float* p = pp + (s + q < A.parts ? s + q : A.parts - 1) * step;
+      a[q] = p[jl];
+      b[q] = p[16 + c * 16 + jl];
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (s + q < A.parts) ss += a[q], d += b[q];
   }
   A.out[e] = d / sqrtf(ss / (float)A.H + A.eps);
 }
@@ -473,18 +496,31 @@ __global__ void k_rs_finish(RsArgs A) {
 
 using namespace dsv;
 
-// H slices of a call: a workgroup a CU, a tile of RS_TH h each at least.
-static int rs_slices(int64_t units, int32_t H) {
-  const int64_t blocks = (units + RS_B / 16 - 1) / (RS_B / 16), tiles = (H + RS_TH - 1) / RS_TH;
-  const int64_t want = blocks >= 256 ? 1 : 256 / blocks;
-  return (int)(want < tiles ? want : tiles);
+// The table's tile and H slices.  256-h tiles of eight waves (one workgroup a CU) where they fill the
+// card; below that 64-h tiles of two waves, two workgroups a CU, which spread a small batch over more
+// of it (15 rows, H 4096, R 512: k_rs_table 25 us against 37; 120 rows, the call 88 us against 118; 240
+// rows, the last batch under the line, 127 against 144).
+struct RsPlan {
+  int tile, slices, hs;
+};
+static RsPlan rs_plan(int64_t units, int32_t H) {
+  const int64_t blocks = (units + RS_B / 16 - 1) / (RS_B / 16);
+  RsPlan p;
+  p.tile = blocks * ((H + 255) / 256) >= 256 ? 256 : 64;
+  const int64_t slots = p.tile == 256 ? 256 : 512, tiles = (H + p.tile - 1) / p.tile;
+  const int64_t want = blocks >= slots ? 1 : slots / blocks;
+  p.slices = (int)(want < tiles ? want : tiles);
+  p.hs = (int)((tiles + p.slices - 1) / p.slices) * p.tile;
+  p.slices = (H + p.hs - 1) / p.hs;  // (none of them empty)
+  return p;
 }
 static int64_t rs_round(int64_t bytes) { return (bytes + 255) / 256 * 256; }
 
-// (a bound that grows with n: a workspace sized for n serves every smaller n.  units * slices is at
-// most units * tiles, and at most 8 * 256 while there is more than one slice)
+// (a bound that grows with n: a workspace sized for n serves every smaller n.  A unit leaves a partial
+// sum for every 64 h of a slice's tile: units * parts is at most units * H / 64, and at most 8 * 256 * 4
+// while there is more than one slice)
 extern "C" int64_t dsv_rs_table_workspace_bytes(int64_t n, int32_t K, int32_t H, int32_t R) {
-  const int64_t KB = (K + 15) / 16, units = n * KB, tiles = (H + RS_TH - 1) / RS_TH;
+  const int64_t KB = (K + 15) / 16, units = n * KB, tiles = (H + 255) / 256;
   int64_t us = units * tiles < 2048 ? units * tiles : 2048;
   if (us < units) us = units;
   return rs_round(n * K * R * 6) + rs_round((int64_t)H * R * 6) + 4 * us * (16 + 16 * KB * 16) * 4 + 256;
@@ -543,24 +579,31 @@ extern "C" int dsv_rs_table(const void* raw, int64_t raw_stride, const float* rm
   A.sqrt_c = (float)sqrt((double)C);
   A.KB = (K + 15) / 16;
   A.units = (int32_t)n * A.KB;
-  A.slices = rs_slices(A.units, H);
-  A.hs = ((H + RS_TH - 1) / RS_TH + A.slices - 1) / A.slices * RS_TH;
-  A.slices = (H + A.hs - 1) / A.hs;  // (none of them empty)
+  const RsPlan plan = rs_plan(A.units, H);
+  A.hs = plan.hs;
+  A.parts = plan.slices * (plan.tile / 64);
   char* ws = reinterpret_cast<char*>(rs_round((int64_t)workspace));  // (16-byte copies; the size has 256 spare)
   A.msg = reinterpret_cast<uint16_t*>(ws);
   A.wsplit = reinterpret_cast<uint16_t*>(ws + rs_round(n * K * R * 6));
   A.part = reinterpret_cast<float*>(ws + rs_round(n * K * R * 6) + rs_round((int64_t)H * R * 6));
   A.out = out;
-  const int64_t Ns = n * K;
-  hipLaunchKernelGGL(k_rs_message, dim3((unsigned)((Ns + RS_B - 1) / RS_B), (unsigned)(R / 64)), dim3(256), 0, stream, A);
-  hipLaunchKernelGGL(k_rs_split, dim3((unsigned)(((int64_t)H * R / 8 + 255) / 256)), dim3(256), 0, stream, A);
-  DSV_CHECK_LAUNCH("k_rs_message / k_rs_split");
-  const dim3 tg((unsigned)((A.units + RS_B / 16 - 1) / (RS_B / 16)), (unsigned)A.slices);
+  // 64 message columns a workgroup where that fills the card, 16 below (15 rows: 21 us against 44)
+  A.sblocks = (int32_t)((n * K + RS_B - 1) / RS_B);
+  const int rc = A.sblocks * (R / 64) >= 256 ? 64 : 16;
+  const dim3 mg((unsigned)(A.sblocks * (R / rc) + ((int64_t)H * R / 8 + 255) / 256));
+  if (rc == 64) hipLaunchKernelGGL(k_rs_message<64>, mg, dim3(256), 0, stream, A);
+  else hipLaunchKernelGGL(k_rs_message<16>, mg, dim3(256), 0, stream, A);
+  DSV_CHECK_LAUNCH("k_rs_message");
+  const dim3 tg((unsigned)((A.units + RS_B / 16 - 1) / (RS_B / 16)), (unsigned)plan.slices);
+  auto table = [&](auto wide, auto narrow) {
+    if (plan.tile == 256) hipLaunchKernelGGL(wide, tg, dim3(512), 0, stream, A);
+    else hipLaunchKernelGGL(narrow, tg, dim3(128), 0, stream, A);
+  };
   switch (A.KB) {
-    case 1: hipLaunchKernelGGL(k_rs_table<1>, tg, dim3(512), 0, stream, A); break;
-    case 2: hipLaunchKernelGGL(k_rs_table<2>, tg, dim3(512), 0, stream, A); break;
-    case 3: hipLaunchKernelGGL(k_rs_table<3>, tg, dim3(512), 0, stream, A); break;
-    default: hipLaunchKernelGGL(k_rs_table<4>, tg, dim3(512), 0, stream, A); break;
+    case 1: table(k_rs_table<1, 256>, k_rs_table<1, 64>); break;
+    case 2: table(k_rs_table<2, 256>, k_rs_table<2, 64>); break;
+    case 3: table(k_rs_table<3, 256>, k_rs_table<3, 64>); break;
+    default: table(k_rs_table<4, 256>, k_rs_table<4, 64>); break;
   }
   DSV_CHECK_LAUNCH("k_rs_table");
   const int64_t total = n * K * K;

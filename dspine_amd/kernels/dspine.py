@@ -137,7 +137,7 @@ def serial_rs_table(raw, rms, query, anchors, cand, codebook, pred_gate_w, prev_
     ``res_emb[s] @ res_proj^T``), ``e = sqrt(C) * codebook[s]`` for sender ``s`` (the anchor on a
     request's first block row, else candidate j of the previous row), ``x``, ``scale``, ``q`` the
     row's pre-write state, write scale and receiver query.  Float32 accuracy on the bf16 matrix cores
-    in four launches (``dsv_rs_table``); ``chunk_rows`` is accepted for the reference's signature (nothing
+    in three launches (``dsv_rs_table``); ``chunk_rows`` is accepted for the reference's signature (nothing
     is chunked: no intermediate of the size it bounds is materialised).
 
     raw [bs*T, H], query [bs*T, >= R], codebook [V, C], lm_head_w [V, H], candidate_head
