@@ -3477,42 +3477,61 @@ __global__ __launch_bounds__(CT) void k_prob_prep(const float* __restrict__ prob
 // ---------------------------------------------------------------------------------------
 // Greedy verify (verification/caps.py:32-59, verification/ragged.py:51-76)
 // ---------------------------------------------------------------------------------------
-__device__ inline int64_t chunk_argmax(const ChunkStat* cs, int C) {
+// First argmax of a row from its chunks' maxima, by a wave: the first chunk holding the largest (0 if
+// none exceeds -inf).
+__device__ __forceinline__ int32_t chunk_argmax(const ChunkStat* cs, int C, int lane) {
   float M = -INFINITY;
-  int32_t arg = INT_MAX;
-  for (int c = 0; c < C; ++c)
-    if (cs[c].m > M) {
-      M = cs[c].m;
-      arg = cs[c].arg;
-    }
-  return arg == INT_MAX ? 0 : arg;
+  int32_t arg = 0;
+  for (int c0 = 0; c0 < C; c0 += WAVE) {
+    const bool in = c0 + lane < C;
+    const ChunkStat* s = cs + (in ? c0 + lane : 0);
+    const float m = in ? s->m : -INFINITY;
+    const int32_t at = s->arg;
+    const float mx = wave_max_f32(m);
+    if (!(mx > M)) continue;
+    M = mx;
+    arg = readlane_at(at, __ffsll((unsigned long long)__ballot(m == mx)) - 1);
+  }
+  return arg;
 }
 
-__global__ void k_greedy_accept(const ChunkStat* cstat, int C, const int64_t* cand, const int32_t* lens,
-                                int32_t cap_static, const int32_t* prefix, int32_t bs, int32_t T,
-                                int32_t* accept, int32_t* commit, int64_t* bonus, int64_t* output,
-                                int32_t* new_seq, int64_t* top1_out) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= bs) return;
+// Greedy acceptance, one workgroup per request, a wave per row: every row's argmax at once.  (One lane
+// walking the request's rows and chunks one load after another took 23.6 us at 1 x 17 rows of 13
+// chunks, this 3.0.)
+constexpr int GA_THREADS = 1024;
+constexpr int GA_ROWS = 1024;  // argmaxes kept in LDS
+__global__ __launch_bounds__(GA_THREADS) void k_greedy_accept(const ChunkStat* cstat, int C, const int64_t* cand,
+                                                             const int32_t* lens, int32_t cap_static,
+                                                             const int32_t* prefix, int32_t T, int32_t* accept,
+                                                             int32_t* commit, int64_t* bonus, int64_t* output,
+                                                             int32_t* new_seq, int64_t* top1_out) {
+  __shared__ int32_t top1[GA_ROWS];
+  __shared__ int s_acc;
+  const int64_t b = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
   int cap = lens ? lens[b] : cap_static;
   cap = cap < 1 ? 1 : (cap > T ? T : cap);
-  int acc = cap - 1;
-  for (int i = 0; i < cap - 1; ++i) {
-    if (cand[(int64_t)b * T + i + 1] != chunk_argmax(cstat + ((int64_t)b * T + i) * C, C)) {
-      acc = i;
-      break;
-    }
+  if (tid == 0) s_acc = cap - 1;
+  __syncthreads();
+  const int rows = top1_out ? T : cap;
+  for (int i = w; i < rows; i += GA_THREADS / WAVE) {
+    const int32_t arg = chunk_argmax(cstat + (b * T + i) * C, C, lane);
+    if (lane) continue;
+    if (i < GA_ROWS) top1[i] = arg;
+    if (top1_out) top1_out[b * T + i] = arg;
+    if (i < cap - 1 && cand[b * T + i + 1] != arg) atomicMin(&s_acc, i);
   }
-  const int64_t bon = chunk_argmax(cstat + ((int64_t)b * T + acc) * C, C);
-  for (int i = 0; i < T; ++i) {
-    const int64_t proposed = i < T - 1 ? cand[(int64_t)b * T + i + 1] : 0;
-    output[(int64_t)b * T + i] = i == acc ? bon : proposed;
-    if (top1_out) top1_out[(int64_t)b * T + i] = chunk_argmax(cstat + ((int64_t)b * T + i) * C, C);
+  __syncthreads();
+  const int acc = s_acc;
+  const int64_t bon = acc < GA_ROWS ? top1[acc] : chunk_argmax(cstat + (b * T + acc) * C, C, lane);
+  for (int i = tid; i < T; i += GA_THREADS)
+    output[b * T + i] = i == acc ? bon : (i < T - 1 ? cand[b * T + i + 1] : 0);
+  if (tid == 0) {
+    accept[b] = acc;
+    commit[b] = acc + 1;
+    bonus[b] = bon;
+    new_seq[b] = prefix[b] + acc + 1;
   }
-  accept[b] = acc;
-  commit[b] = acc + 1;
-  bonus[b] = bon;
-  new_seq[b] = prefix[b] + acc + 1;
 }
 
 // Top-k API: merge chunk candidate lists of each row (one workgroup per row).
@@ -3957,8 +3976,8 @@ static int greedy_launch(const void* logits, int32_t dtype, int64_t rows, int64_
   if (prof && hipEventRecord(g_prof_stop, stream) != hipSuccess)
     DSV_FAIL(DSV_ERR_LAUNCH, "dsv_greedy_verify: cannot record the profiling stop event");
   DSV_CHECK_LAUNCH("k_chunk");
-  hipLaunchKernelGGL(k_greedy_accept, dim3((bs + 63) / 64), dim3(64), 0, stream, P.cstat, P.C, candidates,
-                     verify_lens, cap, prefix_lens, bs, T, accept, commit, bonus, output, new_seq, top1_out);
+  hipLaunchKernelGGL(k_greedy_accept, dim3((unsigned)bs), dim3(GA_THREADS), 0, stream, P.cstat, P.C, candidates,
+                     verify_lens, cap, prefix_lens, T, accept, commit, bonus, output, new_seq, top1_out);
   DSV_CHECK_LAUNCH("k_greedy_accept");
   return DSV_OK;
 }

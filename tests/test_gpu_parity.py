@@ -185,6 +185,32 @@ def test_greedy_ties_and_caps(device, dtype):
             assert np.array_equal(got.cpu().numpy(), r), (cap, vl)
 
 
+@pytest.mark.parametrize("bs,T,V,dtype", [(2, 1, 64, torch.float32), (3, 17, 1 << 20, torch.bfloat16),
+                                          (2, 1100, 40, torch.float32)])
+def test_greedy_edges(device, bs, T, V, dtype):
+    """A block without drafts, rows of more than 32 chunks, and more rows than the accept kernel
+    keeps argmaxes of; with the optional argmaxes and without."""
+    from dspine_amd.verification.caps import accept_greedy
+
+    O = _oracle()
+    g = torch.Generator().manual_seed(T)
+    logits = torch.randint(-60, 60, (bs * T, V), generator=g).to(dtype)
+    logits[0] = -float("inf")  # nothing above -inf: the first id
+    top1 = O.argmax_rows(logits)
+    cand = torch.zeros(bs, T, dtype=torch.int64)
+    cand[:, 1:] = torch.as_tensor(top1).view(bs, T)[:, : T - 1]
+    if T > 2:
+        cand[1, T - 1] = (cand[1, T - 1] + 1) % V
+    prefix = torch.arange(bs, dtype=torch.int32)
+    ref = O.greedy_accept(top1, cand.numpy(), [T] * bs, prefix.numpy())
+    for top in (None, torch.full((bs, T), -1, dtype=torch.int64, device=device)):
+        outs = accept_greedy(candidates=cand.to(device), next_token_logits=logits.to(device),
+                             prefix_lens=prefix.to(device), cap=T, top1=top)
+        for got, r in zip(outs, ref):
+            assert np.array_equal(got.cpu().numpy(), r)
+        assert top is None or np.array_equal(top.cpu().numpy().reshape(-1), np.asarray(top1).reshape(-1))
+
+
 # ------------------------------------------------------------------------------------------
 # fused sampled verify
 # ------------------------------------------------------------------------------------------
