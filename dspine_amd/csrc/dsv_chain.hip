@@ -878,19 +878,16 @@ __global__ __launch_bounds__(WAVE) void k_pack_joint(const float* top_vals, cons
   const float tp = top_ps[r];
   float higher = 0.f;  // mass of strictly larger p, in rank order
   for (int j = 0; j < W; ++j) {
-    const float pj = __shfl(p, j, WAVE);
+    const float pj = readlane_at(p, j);
     higher += pj > p ? pj : 0.f;
   }
   const bool keep = live && p > 0.f && p >= threshold && (higher < tp || tp >= 1.f);
   const uint64_t kept = __ballot(keep);
   const int count = __popcll(kept);
   float total = 0.f;  // the kept mass, summed in rank order
-  for (int j = 0; j < W; ++j) {
-    const float pj = __shfl(p, j, WAVE);
-    total += ((kept >> j) & 1ull) ? pj : 0.f;
-  }
+  for (int j = 0; j < W; ++j) total += ((kept >> j) & 1ull) ? readlane_at(p, j) : 0.f;
   int rank = 0;  // position among the kept ids in ascending id order
-  for (int j = 0; j < W; ++j) rank += ((kept >> j) & 1ull) && __shfl(id, j, WAVE) < id;
+  for (int j = 0; j < W; ++j) rank += ((kept >> j) & 1ull) && readlane_at(id, j) < id;
   if (keep && rank < capacity) {
     ids[r * capacity + rank] = (int32_t)id;
     values[r * capacity + rank] = p / total;
@@ -905,11 +902,20 @@ __global__ __launch_bounds__(WAVE) void k_pack_joint(const float* top_vals, cons
   }
 }
 
-// Overflow rows of the sparse joint target: P[r] = p * (p >= p[k-1]) / sum, in place.
-__global__ __launch_bounds__(CMP_THREADS) void k_overflow_dense(const float* top_vals, int32_t W,
-                                                               const int32_t* top_ks, const int32_t* overflow,
-                                                               float* P, int64_t vocab, int64_t p_stride) {
-  constexpr int NW = CMP_THREADS / WAVE;
+// Overflow rows of the sparse joint target: P[r] = p * (p >= p[k-1]) / sum, in place, one workgroup a
+// row: a pass for the sum, one that writes.  A row is bound by what one CU keeps in flight: 16 waves
+// with eight 16-byte loads a thread (62 us at 24 x 16 rows of 151936, a third of them overflowing, against 246 with 512 threads
+// and one 4-byte load each).  Nearly every vector holds nothing kept and is written as zeros; the
+// division is left to the vectors that do.
+constexpr int OV_THREADS = 1024;
+constexpr int OV_VECS = 8;
+typedef float ovf4 __attribute__((ext_vector_type(4)));
+typedef ovf4 ovf4u __attribute__((aligned(4)));  // (rows of any stride)
+
+__global__ __launch_bounds__(OV_THREADS) void k_overflow_dense(const float* top_vals, int32_t W,
+                                                              const int32_t* top_ks, const int32_t* overflow,
+                                                              float* P, int64_t vocab, int64_t p_stride) {
+  constexpr int NW = OV_THREADS / WAVE;
   __shared__ double red[NW];
   const int64_t r = blockIdx.x;
   if (overflow[r] == 0) return;
@@ -917,16 +923,38 @@ __global__ __launch_bounds__(CMP_THREADS) void k_overflow_dense(const float* top
   k = k < 1 ? 1 : (k > W ? W : k);
   const float threshold = top_vals[r * W + k - 1];
   float* row = P + r * p_stride;
+  const int tid = threadIdx.x;
+  const int64_t nv = vocab / 4;  // whole vectors; the last vocab % 4 values are thread 0..2's
+  const int64_t tail = 4 * nv + tid;
+  auto each = [&](auto&& f) {  // f(vector index, value) over this thread's vectors, OV_VECS loads in flight
+    for (int64_t v0 = tid; v0 < nv; v0 += (int64_t)OV_VECS * OV_THREADS) {
+      ovf4 x[OV_VECS];
+#pragma unroll
+      for (int e = 0; e < OV_VECS; ++e) {
+        const int64_t v = v0 + (int64_t)e * OV_THREADS;
+        x[e] = *reinterpret_cast<const ovf4u*>(row + 4 * (v < nv ? v : v0));
+      }
+#pragma unroll
+      for (int e = 0; e < OV_VECS; ++e)
+        if (v0 + (int64_t)e * OV_THREADS < nv) f(v0 + (int64_t)e * OV_THREADS, x[e]);
+    }
+  };
   double s = 0.0;
-  for (int64_t j = threadIdx.x; j < vocab; j += CMP_THREADS) {
-    const float x = row[j];
-    s += x >= threshold ? (double)x : 0.0;
-  }
+  each([&](int64_t, const ovf4& x) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) s += x[c] >= threshold ? (double)x[c] : 0.0;
+  });
+  if (tail < vocab && row[tail] >= threshold) s += (double)row[tail];
   const float total = (float)block_sum<NW>(s, red);
-  for (int64_t j = threadIdx.x; j < vocab; j += CMP_THREADS) {
-    const float x = row[j];
-    row[j] = x >= threshold ? x / total : 0.f;
-  }
+  each([&](int64_t v, const ovf4& x) {
+    ovf4 y = {0.f, 0.f, 0.f, 0.f};
+    if (x[0] >= threshold || x[1] >= threshold || x[2] >= threshold || x[3] >= threshold) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) y[c] = x[c] >= threshold ? x[c] / total : 0.f;
+    }
+    *reinterpret_cast<ovf4u*>(row + 4 * v) = y;
+  });
+  if (tail < vocab) row[tail] = row[tail] >= threshold ? row[tail] / total : 0.f;
 }
 
 }  // namespace dsv
@@ -1138,7 +1166,7 @@ extern "C" int dsv_pack_joint(const float* top_vals, const int64_t* top_ids, int
                      capacity, ids, values, lengths, overflow);
   DSV_CHECK_LAUNCH("dsv_pack_joint");
   if (P) {
-    hipLaunchKernelGGL(k_overflow_dense, dim3((unsigned)rows), dim3(CMP_THREADS), 0, stream, top_vals, W, top_ks,
+    hipLaunchKernelGGL(k_overflow_dense, dim3((unsigned)rows), dim3(OV_THREADS), 0, stream, top_vals, W, top_ks,
                        overflow, P, vocab, p_stride);
     DSV_CHECK_LAUNCH("dsv_pack_joint");
   }

@@ -466,6 +466,30 @@ def test_build_sparse_target(device, capacity):
     assert build_sparse_target(logits.to(device), W.info_to(info, device), block_size=T, capacity=capacity) is None
 
 
+@pytest.mark.parametrize("V", [33, 4093, 32771, 40004])
+def test_overflow_rows_dense(device, V):
+    """Overflow rows renormalised in place at the edges of the pass's vectors and rounds (1024 threads x
+    4 values x 8 loads), between rows that stay as they are."""
+    from dspine_amd.sampling.sparse.target import build_sparse_target
+
+    O = _O()
+    g = torch.Generator().manual_seed(V)
+    rows = 5
+    logits = torch.randn(rows, V, generator=g)
+    for r in (0, 2, 4):  # ties at the k-th place, the row's last ids among them
+        logits[r, torch.randperm(V, generator=g)[:20]] = 6.0
+        logits[r, V - 7:] = 6.0
+        logits[r, 1] = 7.0
+    ks, ps = torch.full((rows,), 8), torch.ones(rows)
+    info = W.sampling_info(torch.ones(rows), ks, ps)
+    info.is_any_greedy = False
+    st = build_sparse_target(logits.to(device), W.info_to(info, device), block_size=1, capacity=16)
+    p = O.softmax_temp(logits, torch.ones(rows), exact=True)
+    _, _, _, ovf, dense = O.sparse_target(p, ks, ps, 16)
+    assert ovf.tolist() == [1, 0, 1, 0, 1] and torch.equal(st.packed[3].cpu(), ovf)
+    torch.testing.assert_close(st.dense_p.cpu(), dense, rtol=1e-5, atol=1e-9)
+
+
 # ------------------------------------------------------------------------------------------
 # logit adjustments (sampling/compact.py:14-79), padding, window index
 # ------------------------------------------------------------------------------------------
