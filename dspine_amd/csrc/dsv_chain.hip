@@ -787,72 +787,168 @@ __global__ __launch_bounds__(CH_THREADS) void k_chain(dsv_chain_args a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Draft-side K-lane chain (kernels/dspine.py:616-674): one wave per request walks its T-1 rows
-// of the [K, K] table; lanes are the K candidates.
+// Draft-side K-lane chain (kernels/dspine.py:616-674): a request's T-1 block rows, lanes the K
+// candidates, one workgroup per request.  A row's draw depends on the chain only through its sender,
+// the lane drawn on the row before.  Up to 16 lanes the workgroup evaluates every (row, sender) pair at
+// once (G lanes each, G the power of two from K up), walks the drawn lanes through LDS, and evaluates
+// the walked pairs again for the outputs.  Wider tables have too many pairs for that: their rows are
+// brought to LDS in batches and one wave walks them.  Bound by latency: a wave walking the rows from
+// memory took 46 us at 64 requests of 15 rows of 16 lanes (3 us a row) and 70 us at 16 rows of 32, this
+// 14 and 54; evaluating every pair at 32 lanes was slower than the wave's walk (the round's four calls
+// 104 us against 89).
 // ---------------------------------------------------------------------------------------
-__global__ __launch_bounds__(WAVE) void k_sample_chain(const float* table, int32_t K, int32_t tm1,
-                                                      const float* inv_temp, const int32_t* top_k,
-                                                      const float* top_p, const float* min_p, const int32_t* greedy,
-                                                      const float* u, const int64_t* cand, const int64_t* greedy_tok,
-                                                      int64_t* out_tok, float* out_q, float* confidence) {
-  const int b = blockIdx.x;
-  const int lane = threadIdx.x;
-  const bool live = lane < K;
-  const float inv_t = inv_temp[b];
+constexpr int SC_THREADS = 1024;
+constexpr int SC_PAIRS = 8192;  // (row, sender) pairs a batch holds
+constexpr int SC_TILE = 16384;  // table values a batch of the walk holds (a row of 64 lanes: 4096)
+
+struct ScDraw {
+  float q, pmax;
+  int choice;
+};
+// The maximum over each group of G lanes (G = 32, 64: over the wave, whose groups hold the same).
+template <int G>
+__device__ __forceinline__ float sc_max(float v) {
+  if constexpr (G > 16) return wave_max_f32(v);
+  v = fmaxf(v, dpp<DPP_QUAD_XOR1>(v, v));
+  v = fmaxf(v, dpp<DPP_QUAD_XOR2>(v, v));
+  v = fmaxf(v, dpp<DPP_ROW_HALF_MIRROR>(v, v));
+  if constexpr (G == 16) v = fmaxf(v, dpp<DPP_ROW_MIRROR>(v, v));
+  return v;
+}
+
+// One pair's draw by a group of G lanes: q of this lane, max p, the drawn lane.  (The sums run in the
+// lane order of a 64-lane tree whose upper lanes hold nothing.)
+template <int G>
+__device__ __forceinline__ ScDraw sc_draw(float score, int l, int K, int32_t tk, float tp, float mp, float u) {
+  const bool live = l < K;
+  const float mx = sc_max<G>(score);  // (by every lane: it moves values between them)
+  const float mass = live ? expf(score - mx) : 0.f;
+  float tot = mass;
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) tot += __shfl_xor(tot, o, G);
+  const float p = live ? mass / tot : -1.f;
+  const float pmax = sc_max<G>(p);
+  // rank and mass ahead (ties: lower lane first)
+  int rank = 0;
+  float before = 0.f;
+#pragma unroll
+  for (int d = 0; d < G; ++d) {  // (a lane past K holds -1: ahead of none)
+    const float pd = __shfl(p, d, G);
+    const bool ahead = pd > p || (pd == p && d < l);
+    rank += ahead;
+    before += ahead ? pd : 0.f;
+  }
+  const bool keep = live && rank < tk && before <= tp && p >= mp * pmax;
+  const float w = keep ? p : 0.f;
+  float ws = w;
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) ws += __shfl_xor(ws, o, G);
+  const float q = live ? w / ws : 0.f;
+  // inclusive prefix of q in lane order
+  float cdf = q;
+#pragma unroll
+  for (int o = 1; o < G; o <<= 1) {
+    const float t = __shfl_up(cdf, o, G);
+    if (l >= o) cdf += t;
+  }
+  const float threshold = u * __shfl(cdf, K - 1, G);
+  const int base = threadIdx.x & (WAVE - 1) & ~(G - 1);
+  constexpr uint64_t M = G == 64 ? ~0ull : (1ull << (G & 63)) - 1;
+  const uint64_t under = (__ballot(live && cdf <= threshold) >> base) & M, kept = (__ballot(keep) >> base) & M;
+  const int choice = __popcll(under), last = kept ? 63 - __clzll((long long)kept) : 0;
+  return {q, pmax, choice < last ? choice : last};
+}
+
+template <int G>
+__global__ __launch_bounds__(SC_THREADS) void k_sample_chain(const float* table, int32_t K, int32_t tm1,
+                                                            const float* inv_temp, const int32_t* top_k,
+                                                            const float* top_p, const float* min_p,
+                                                            const int32_t* greedy, const float* u,
+                                                            const int64_t* cand, const int64_t* greedy_tok,
+                                                            int64_t* out_tok, float* out_q, float* confidence) {
+  constexpr int NG = SC_THREADS / G;
+  const int64_t b = blockIdx.x, n0 = b * tm1;
+  const int tid = threadIdx.x, grp = tid / G, l = tid % G;
+  if (greedy[b] != 0) {  // greedy_tok with a one-hot q; the chain is not read
+    for (int64_t e = tid; e < (int64_t)tm1 * K; e += SC_THREADS) {
+      const int64_t n = n0 + e / K;
+      out_q[n * K + e % K] = cand[n * K + e % K] == greedy_tok[n] ? 1.f : 0.f;
+      if (e % K == 0) out_tok[n] = greedy_tok[n];
+    }
+    return;
+  }
+  const float inv_t = inv_temp[b], tp = top_p[b], mp = min_p[b];
   const int32_t tk = top_k[b];
-  const float tp = top_p[b];
-  const float mp = min_p[b];
-  const bool gr = greedy[b] != 0;
-  int sender = 0;
-  for (int i = 0; i < tm1; ++i) {
-    const int64_t n = (int64_t)b * tm1 + i;
-    const float score = live ? table[(n * K + sender) * K + lane] * inv_t : -INFINITY;
-    float mx = score;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, WAVE));
-    const float mass = live ? expf(score - mx) : 0.f;
-    float tot = mass;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o, WAVE);
-    const float p = live ? mass / tot : -1.f;
-    float pmax = p;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) pmax = fmaxf(pmax, __shfl_xor(pmax, o, WAVE));
-    if (confidence && !gr && lane == 0) confidence[n] = pmax;
-    // rank and mass ahead (ties: lower lane first)
-    int rank = 0;
-    float before = 0.f;
-    for (int d = 0; d < K; ++d) {
-      const float pd = __shfl(p, d, WAVE);
-      const bool ahead = pd > p || (pd == p && d < lane);
-      rank += ahead;
-      before += ahead ? pd : 0.f;
+  const int lc = l < K ? l : K - 1;
+  if constexpr (G > 16) {
+    __shared__ float tile[SC_TILE], us[SC_TILE / 256];
+    __shared__ uint8_t drawn[SC_TILE / 256];  // (K > 16: at most SC_TILE / 289 rows a batch)
+    const int batch = SC_TILE / (K * K);
+    int sender = 0;
+    for (int i0 = 0; i0 < tm1; i0 += batch) {
+      const int rows = tm1 - i0 < batch ? tm1 - i0 : batch;
+      for (int e = tid; e < rows * K * K; e += SC_THREADS) tile[e] = table[(n0 + i0) * K * K + e];
+      if (tid < rows) us[tid] = u[n0 + i0 + tid];
+      __syncthreads();
+      if (tid < WAVE) {
+        for (int i = 0; i < rows; ++i) {
+          const int64_t n = n0 + i0 + i;
+          const float x = __fmul_rn(tile[(i * K + sender) * K + lc], inv_t);
+          const ScDraw d = sc_draw<G>(l < K ? x : -INFINITY, l, K, tk, tp, mp, us[i]);
+          if (tid < K) out_q[n * K + l] = d.q;
+          if (tid == 0) {
+            drawn[i] = (uint8_t)d.choice;
+            if (confidence) confidence[n] = d.pmax;
+          }
+          sender = d.choice;
+        }
+      }
+      __syncthreads();
+      if (tid < rows) out_tok[n0 + i0 + tid] = cand[(n0 + i0 + tid) * K + drawn[tid]];
+      __syncthreads();
     }
-    const bool keep = live && rank < tk && before <= tp && p >= mp * pmax;
-    const float w = keep ? p : 0.f;
-    float ws = w;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) ws += __shfl_xor(ws, o, WAVE);
-    const float q = live ? w / ws : 0.f;
-    // inclusive prefix of q in lane order
-    float cdf = q;
-#pragma unroll
-    for (int o = 1; o < WAVE; o <<= 1) {
-      const float t = __shfl_up(cdf, o, WAVE);
-      if (lane >= o) cdf += t;
+    return;
+  }
+  __shared__ uint8_t drawn[SC_PAIRS], senders[SC_PAIRS];
+  __shared__ int s_sender;
+  auto score = [&](int64_t n, int sender) {
+    const float x = __fmul_rn(table[(n * K + sender) * K + lc], inv_t);  // (rounded: not into score - max)
+    return l < K ? x : -INFINITY;
+  };
+  const int batch = SC_PAIRS / K;
+  for (int i0 = 0; i0 < tm1; i0 += batch) {
+    const int rows = tm1 - i0 < batch ? tm1 - i0 : batch, pairs = rows * K;
+    // the next pair's loads in flight under this one's draw
+    float sn = 0.f, un = 0.f;
+    if (grp < pairs) sn = score(n0 + i0 + grp / K, grp % K), un = u[n0 + i0 + grp / K];
+    for (int pr = grp; pr < pairs; pr += NG) {
+      const float sc = sn, uc = un;
+      const int nx = pr + NG < pairs ? pr + NG : pr;
+      sn = score(n0 + i0 + nx / K, nx % K);
+      un = u[n0 + i0 + nx / K];
+      const ScDraw d = sc_draw<G>(sc, l, K, tk, tp, mp, uc);
+      if (l == 0) drawn[pr] = (uint8_t)d.choice;
     }
-    const float total = __shfl(cdf, K - 1, WAVE);
-    const float threshold = u[n] * total;
-    int choice = __popcll(__ballot(live && cdf <= threshold));
-    const uint64_t kept = __ballot(keep);
-    const int last = kept ? 63 - __clzll((long long)kept) : 0;
-    choice = choice < last ? choice : last;
-    const int64_t cl = live ? cand[n * K + lane] : 0;
-    const int64_t sampled = __shfl(cl, choice, WAVE);
-    const int64_t gtok = greedy_tok[n];
-    if (lane == 0) out_tok[n] = gr ? gtok : sampled;
-    if (live) out_q[n * K + lane] = gr ? (cl == gtok ? 1.f : 0.f) : q;
-    sender = choice;
+    __syncthreads();
+    if (tid == 0) {
+      int s = i0 ? s_sender : 0;
+      for (int i = 0; i < rows; ++i) {
+        senders[i] = (uint8_t)s;
+        s = drawn[i * K + s];
+      }
+      s_sender = s;
+    }
+    __syncthreads();
+    for (int i = grp; i < rows; i += NG) {
+      const int64_t n = n0 + i0 + i;
+      const ScDraw d = sc_draw<G>(score(n, senders[i]), l, K, tk, tp, mp, u[n]);
+      if (l < K) out_q[n * K + l] = d.q;
+      if (l == 0) {
+        out_tok[n] = cand[n * K + d.choice];
+        if (confidence) confidence[n] = d.pmax;
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -1143,8 +1239,14 @@ extern "C" int dsv_sample_chain(const float* table, int64_t n, int32_t K, int32_
   const int64_t bs = n / (block_size - 1);
   if (bs == 0) return DSV_OK;
   if (bs > 2147483647ll) DSV_FAIL(DSV_ERR_INVALID, "dsv_sample_chain: too many chains");
-  hipLaunchKernelGGL(k_sample_chain, dim3((unsigned)bs), dim3(WAVE), 0, stream, table, K, block_size - 1, inv_temp,
-                     top_k, top_p, min_p, greedy, u, cand, greedy_tok, out_tok, out_q, confidence);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)bs), dim3(SC_THREADS), 0, stream, table, K, block_size - 1, inv_temp,
+                       top_k, top_p, min_p, greedy, u, cand, greedy_tok, out_tok, out_q, confidence);
+  };
+  if (K <= 8) launch(k_sample_chain<8>);
+  else if (K <= 16) launch(k_sample_chain<16>);
+  else if (K <= 32) launch(k_sample_chain<32>);
+  else launch(k_sample_chain<64>);
   DSV_CHECK_LAUNCH("dsv_sample_chain");
   return DSV_OK;
 }

@@ -663,6 +663,23 @@ def test_sample_chain_matches_oracle(device, seed):
     assert bool((out_q[torch.arange(n), lane] > 0).all())
 
 
+@pytest.mark.parametrize("k,T", [(1, 4), (8, 3), (9, 17), (16, 2), (16, 515), (17, 60), (32, 18), (33, 16), (64, 7)])
+def test_sample_chain_widths(device, k, T):
+    """Every group width (8, 16, 32, 64 lanes) at its edges, chains that fill more than one batch of
+    rows (512 rows of 16 lanes; 56 of 17, 16 of 32, 15 of 33, 4 of 64), a greedy request among them."""
+    O = _O()
+    params = [(1.0, k, 1.0, 0.0, 0), (0.7, max(1, k // 2), 0.8, 0.05, 0), (1.0, k, 1.0, 0.0, 1)]
+    table, cand, greedy_tok, u = _chain_inputs(len(params), T, k, 7 * k + T)
+    staged = _staged(params)
+    conf = torch.full((cand.shape[0],), -0.5, device=device)
+    out_tok, out_q = _run_chain(device, table, staged, u, cand, greedy_tok, T, confidence=conf)
+    conf_ref = np.full(cand.shape[0], -0.5, np.float32)
+    ref_tok, ref_q = O.sample_chain(*_np(table, *staged, u, cand, greedy_tok), T, confidence=conf_ref)
+    assert np.array_equal(out_tok.numpy(), ref_tok)
+    torch.testing.assert_close(out_q, torch.as_tensor(ref_q), rtol=1e-5, atol=1e-6)
+    torch.testing.assert_close(conf.cpu(), torch.as_tensor(conf_ref), rtol=1e-5, atol=1e-6)
+
+
 def test_sample_chain_ties_break_to_lower_lane(device):
     """tests/test_cuda.py:213-232."""
     T, k = 3, 8
