@@ -68,6 +68,10 @@ constexpr int FLAG_SCAN_DRAW = 4;    // dense row whose bonus draw k_final plans
 constexpr int FLAG_TIES_COUNTED = 8; // full-histogram row whose chunks' counts of cut-key values are in rties
 constexpr int SJ_CAP = 32;           // packed capacity of the sparse joint target (sampling/target.py:84-87)
 
+// Row data of the probability filter: float32 probabilities taken as they are, where the other row
+// kernels take logits -- a value's weight is the value, its order the same.
+constexpr int DT_PROB = 3;
+
 template <int DT>
 struct Elems {
   static constexpr int n = DT == DSV_BF16 ? 8 : 4;    // elements per 16-byte vector
@@ -408,10 +412,18 @@ __device__ __forceinline__ float prob_of(float x, float T, float m_f, float invZ
   return expf(xf - m_f) * invZ;
 }
 
+// The weight of a value, in the row's units: its softmax probability, or the given probability.
+template <int DT>
+__device__ __forceinline__ float weight_of(float x, float T, float m_f, float invZ) {
+  if constexpr (DT == DT_PROB) return x;
+  return prob_of(x, T, m_f, invZ);
+}
+
 // P at one value of a dense row (unfiltered, or a nucleus row's kept value): p, renormalised
 // over the kept mass when the row is filtered.
+template <int DT>
 __device__ __forceinline__ double dense_P(const RowSum& rs, float T, float x) {
-  const float p = prob_of(x, T, rs.m_f, rs.invZ);
+  const float p = weight_of<DT>(x, T, rs.m_f, rs.invZ);
   return (rs.mode == M_HIST || rs.norm) ? (double)(p / rs.S_f) : (double)p;
 }
 

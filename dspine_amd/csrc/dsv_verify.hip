@@ -64,8 +64,8 @@ struct KParams {
   uint32_t* req_cnt;      // [bs]: rows merged per request (zeroed by the chunk pass)
   uint32_t* deferred;     // [bs]: 1 until the row merge wrote the request's outputs (set by the chunk pass)
   int32_t only_deferred;  // k_final skips the requests the row merge finished
-  const float* src_p;     // dense target writer with raw_p: kept entries are src_p's values (the
-  int64_t src_stride;     //   probabilities whose logs are the rows: dsv_filter_probs), else NULL
+  int32_t prob;           // the rows are probabilities (DT_PROB kernels)
+  int32_t top_p_raw;      // DT_PROB rows: top-p tests the raw mass ahead (else a share of the row's mass)
 };
 
 __device__ __forceinline__ const char* row_ptr(const dsv_verify_args& a, int64_t r) {
@@ -878,18 +878,18 @@ __device__ __forceinline__ void merge_row(const KParams& P, int64_t r, int b, in
   }
   const float c2 = log2e_over(T);
   // (support-list rows whose filter does not read Z: p up to the factor 1/Z, renormalised below)
-  const bool nz = mode != M_LIST || list_needs_z(a, pre.top_p);
-  const double Z =
-      nz ? wave_sum(m_l > -INFINITY ? s_l * (double)__builtin_amdgcn_exp2f((m_l - M) * c2) : 0.0) : 1.0;
+  const bool nz = DT == DT_PROB || mode != M_LIST || list_needs_z(a, pre.top_p);
+  const double Z = DT == DT_PROB ? wave_sum(s_l)
+                   : nz ? wave_sum(m_l > -INFINITY ? s_l * (double)__builtin_amdgcn_exp2f((m_l - M) * c2) : 0.0) : 1.0;
   const float m_f = M / T;
-  const float invZ = (float)(1.0 / Z);
+  const float invZ = DT == DT_PROB ? 1.f : (float)(1.0 / Z);
   rs.Z = Z;
   rs.m_f = m_f;
   rs.invZ = invZ;
   // the draft token's adjusted logit (recorded by the chunk that holds it)
   const float xt = (tok >= 0 && tok < a.vocab) ? cs[tok / Elems<DT>::chunk].xtok : -INFINITY;
   if (mode == M_UNF) {
-    const float p = (tok >= 0 && tok < a.vocab) ? prob_of(xt, T, m_f, invZ) : 0.f;
+    const float p = (tok >= 0 && tok < a.vocab) ? weight_of<DT>(xt, T, m_f, invZ) : 0.f;
     if (a.filter) {  // filtered request with nothing cut: P = p / sum(p)
       rs.norm = 1;
       rs.S_kept = Z * (double)invZ;
@@ -909,10 +909,10 @@ __device__ __forceinline__ void merge_row(const KParams& P, int64_t r, int b, in
     const bool live = lane < kk;
     const uint64_t pk = live ? ms.top[lane] : 0ull;
     const int32_t id = live ? unpack_id(pk) : INT_MAX;
-    const float p = live ? prob_of(value_of_key<DT>(unpack_key(pk)), T, m_f, invZ) : 0.f;
+    const float p = live ? weight_of<DT>(value_of_key<DT>(unpack_key(pk)), T, m_f, invZ) : 0.f;
     double lo_p, hi_p;
     const double S_all = wave_tiles((double)p, lo_p, hi_p);
-    const float top_p = pre.top_p;
+    const float top_p = DT == DT_PROB && !P.top_p_raw ? (float)((double)pre.top_p * Z) : pre.top_p;
     const float min_p = pre.min_p;
     bool keep;
     if (a.sparse_joint) {
@@ -949,7 +949,7 @@ __device__ __forceinline__ void merge_row(const KParams& P, int64_t r, int b, in
         rs.flags = FLAG_SCAN_DRAW;
         rs.S_kept = S;
         rs.S_f = (float)S;
-        rs.p_draft = (tok >= 0 && tok < a.vocab && key_of<DT>(xt) >= kcut) ? prob_of(xt, T, m_f, invZ) / rs.S_f : 0.f;
+        rs.p_draft = (tok >= 0 && tok < a.vocab && key_of<DT>(xt) >= kcut) ? weight_of<DT>(xt, T, m_f, invZ) / rs.S_f : 0.f;
         const int32_t ok = tok >= 0 ? step_accept_lds(ds, a.K, tok, rs.p_draft, pre.u) : 0;
         if (lane == 0) {
           ro->rs = rs;
@@ -965,7 +965,7 @@ __device__ __forceinline__ void merge_row(const KParams& P, int64_t r, int b, in
           // sequential branch: renormalise over the top-k, top-p on that mass, then min-p
           double lo_a, hi_a;
           wave_tiles(live ? (double)p / S_all : 0.0, lo_a, hi_a);
-          keep = live && lane < pre.top_k && lo_a <= (double)top_p;
+          keep = live && lane < pre.top_k && lo_a <= (double)pre.top_p;
         }
         const float thr = readlane<0>(p) * min_p;
         if (p < thr) keep = false;
@@ -1032,7 +1032,7 @@ __device__ __forceinline__ void nucleus_finish(const KParams& P, int64_t r, int 
                                                float xtok, int64_t tok, int64_t tie_tok, RowOut* ro,
                                                const DrawShared* fq = nullptr, float coin = 0.f) {
   const bool kept = key_of<DT>(xtok) > rs.vcut || (key_of<DT>(xtok) == rs.vcut && tie_tok < (int64_t)rs.ktie);
-  rs.p_draft = (tok >= 0 && tok < P.a.vocab && kept) ? prob_of(xtok, T, rs.m_f, rs.invZ) / rs.S_f : 0.f;
+  rs.p_draft = (tok >= 0 && tok < P.a.vocab && kept) ? weight_of<DT>(xtok, T, rs.m_f, rs.invZ) / rs.S_f : 0.f;
   int32_t ok = 0;
   if (tok >= 0) ok = fq ? step_accept_lds(*fq, P.a.K, tok, rs.p_draft, coin) : step_accept_wave(P.a, b, s, tok, rs.p_draft);
   if (threadIdx.x == 0) {
@@ -1674,6 +1674,7 @@ __device__ __forceinline__ void nuc_row(const KParams& P, int64_t r, uint32_t* h
 constexpr int F32_BINS = 2048, F32_KEYS = 1024;
 constexpr double FX_ONE = 4611686018427387904.0;  // 2^62
 constexpr uint32_t F32_NEG_INF_KEY = 0x007FFFFFu;  // key of -inf; keys at or below it hold no value
+constexpr uint32_t F32_ZERO_KEY = 0x80000000u;     // key of 0: likewise, of probabilities
 struct F32NucLds {
   uint32_t cnt[2][F32_BINS];
   uint64_t mass[2][F32_BINS];
@@ -1692,10 +1693,10 @@ struct F32NucShared {
 
 // One pass over the row: counts (and, levels 0 and 1, masses) of the values whose key matches the
 // level's prefix.  Level 0 also counts the values at the draft token's key before the token.
-template <bool ALIGNED>
+template <int DT, bool ALIGNED>
 __device__ __forceinline__ void f32_pass(const KParams& P, int b, const char* rowp, float pres, float rep, float T,
                                          float m_f, float invZ, int level, uint32_t prefix, F32NucLds& L,
-                                         uint32_t ktok, int64_t tok, uint32_t& tie_before) {
+                                         uint32_t ktok, int64_t tok, uint32_t& tie_before, double fx) {
   const int tid = threadIdx.x;
   const int64_t V = P.a.vocab;
   const bool pen = P.pbits != nullptr;
@@ -1709,7 +1710,7 @@ __device__ __forceinline__ void f32_pass(const KParams& P, int b, const char* ro
   __syncthreads();
   auto count = [&](float x, int64_t j) {
     const uint32_t k = f32_key(x);
-    if (k <= F32_NEG_INF_KEY) return;
+    if (k <= (DT == DT_PROB ? F32_ZERO_KEY : F32_NEG_INF_KEY)) return;
     uint32_t bin;
     if (level == 0) {
       bin = k >> 21;
@@ -1722,7 +1723,7 @@ __device__ __forceinline__ void f32_pass(const KParams& P, int b, const char* ro
       bin = k & (F32_KEYS - 1);
     }
     atomicAdd(&cnt[bin], 1u);
-    if (mass) atomicAdd((unsigned long long*)&mass[bin], (unsigned long long)((double)prob_of(x, T, m_f, invZ) * FX_ONE));
+    if (mass) atomicAdd((unsigned long long*)&mass[bin], (unsigned long long)((double)weight_of<DT>(x, T, m_f, invZ) * fx));
   };
   constexpr int U = 4;
   const int64_t ve = ALIGNED ? V / 4 : (V + 3) / 4;
@@ -1789,9 +1790,10 @@ __device__ __forceinline__ void f32_prefix(F32NucLds& L, int level, F32NucShared
 // The first non-empty bin of a level after descending rank `after` (rank = 2047 - bin) -- with
 // `test`, the first one that can hold the cut given the values and mass ahead of the level
 // (base_c, base_m).  Returns the bin, -1 for none.
+template <int DT>
 __device__ __forceinline__ int f32_next(const F32NucLds& L, int level, int after, bool test, uint32_t prefix,
                                         uint64_t base_c, uint64_t base_m, float T, float m_f, float invZ, int backend,
-                                        int topk, float min_p, float thr_minp, float top_p, F32NucShared& sh) {
+                                        int topk, float min_p, float thr_minp, float top_p, double fx, F32NucShared& sh) {
   const int tid = threadIdx.x;
   if (tid == 0) sh.best = INT_MAX;
   __syncthreads();
@@ -1805,9 +1807,9 @@ __device__ __forceinline__ int f32_next(const F32NucLds& L, int level, int after
     if (test) {
       uint32_t klo = level == 0 ? (uint32_t)bin << 21 : (prefix << 21) | ((uint32_t)bin << 10);
       if (klo <= F32_NEG_INF_KEY) klo = F32_NEG_INF_KEY + 1u;
-      const float p_lo = prob_of(key_to_f32(klo), T, m_f, invZ);
+      const float p_lo = weight_of<DT>(key_to_f32(klo), T, m_f, invZ);
       const uint64_t n_ge = base_c + L.pcnt[level][bin] + cb;
-      const double S_ge = (double)(base_m + L.pmass[level][bin] + L.mass[level][bin]) / FX_ONE;
+      const double S_ge = (double)(base_m + L.pmass[level][bin] + L.mass[level][bin]) / fx;
       ok = (min_p > 0.f && p_lo < thr_minp) || (n_ge - 1 >= (uint64_t)(topk > 0 ? topk : 0)) ||
            topp_fails(backend, S_ge - (double)p_lo, p_lo, top_p);
     }
@@ -1822,9 +1824,10 @@ __device__ __forceinline__ int f32_next(const F32NucLds& L, int level, int after
 
 // The exact keys of one level-1 bin in descending order: the first key with a failing tie.
 // Returns true with the cut in sh (key, tie, mass ahead of the cut).
+template <int DT>
 __device__ __forceinline__ bool f32_walk(const F32NucLds& L, uint32_t prefix, uint64_t base_c, uint64_t base_m,
                                          float T, float m_f, float invZ, int backend, int topk, float min_p,
-                                         float thr_minp, float top_p, F32NucShared& sh) {
+                                         float thr_minp, float top_p, double fx, F32NucShared& sh) {
   const int tid = threadIdx.x;
   uint32_t c[2];
   float pk[2];
@@ -1834,7 +1837,7 @@ __device__ __forceinline__ bool f32_walk(const F32NucLds& L, uint32_t prefix, ui
   for (int e = 0; e < 2; ++e) {
     const uint32_t lo = (uint32_t)(F32_KEYS - 1 - 2 * tid - e);
     c[e] = L.cnt3[lo];
-    pk[e] = c[e] ? prob_of(key_to_f32((prefix << 10) | lo), T, m_f, invZ) : 0.f;
+    pk[e] = c[e] ? weight_of<DT>(key_to_f32((prefix << 10) | lo), T, m_f, invZ) : 0.f;
     m += (double)c[e] * (double)pk[e];
     n += c[e];
   }
@@ -1844,7 +1847,7 @@ __device__ __forceinline__ bool f32_walk(const F32NucLds& L, uint32_t prefix, ui
   const double mb = block_excl_scan<NUC_WAVES>(m, sh.d, &tm);
   if (tid == 0) sh.best = INT_MAX;
   __syncthreads();
-  double Sb = (double)base_m / FX_ONE + mb;
+  double Sb = (double)base_m / fx + mb;
   uint64_t Nb = base_c + nb;
   int32_t my_tie = 0;
   uint32_t my_key = 0;
@@ -1876,7 +1879,7 @@ __device__ __forceinline__ bool f32_walk(const F32NucLds& L, uint32_t prefix, ui
   return found;
 }
 
-template <bool ALIGNED>
+template <int DT, bool ALIGNED>
 __device__ __forceinline__ void nuc_row_f32(const KParams& P, int64_t r, F32NucLds& L, F32NucShared& sh,
                                             RowOut* ro) {
   const dsv_verify_args& a = P.a;
@@ -1886,12 +1889,14 @@ __device__ __forceinline__ void nuc_row_f32(const KParams& P, int64_t r, F32NucL
   RowSum rs = P.rowsum[r];
   const int64_t V = a.vocab;
   const char* rowp = row_ptr(a, r);
-  const float T = a.temperatures[b];
+  const float T = DT == DT_PROB ? 1.f : a.temperatures[b];
   const int topk = a.top_ks[b];
   const bool pen = P.pbits != nullptr;
   const float pres = pen && a.presence ? a.presence[b] : 0.f;
   const float rep = pen && a.repetition ? a.repetition[b] : 1.f;
-  const float top_p = a.top_ps[b];
+  // (the fixed point: 2^62 to the row's mass, 1 for a softmax, to within a factor of two)
+  const double fx = DT == DT_PROB && rs.Z > 0.0 && rs.Z < 1e300 ? ldexp(1.0, 61 - ilogb(rs.Z)) : FX_ONE;
+  const float top_p = a.top_ps[b] * (DT == DT_PROB && !P.top_p_raw ? (float)rs.Z : 1.f);
   const float min_p = (a.need_min_p && a.min_ps) ? a.min_ps[b] : 0.f;
   const int64_t tok = step_token(a, b, s);
   float xt = -INFINITY;
@@ -1901,9 +1906,9 @@ __device__ __forceinline__ void nuc_row_f32(const KParams& P, int64_t r, F32NucL
   }
   const uint32_t ktok = f32_key(xt);
   const float m_f = rs.m_f, invZ = rs.invZ;
-  const float thr_minp = prob_of(key_to_f32(rs.kmax), T, m_f, invZ) * min_p;
+  const float thr_minp = weight_of<DT>(key_to_f32(rs.kmax), T, m_f, invZ) * min_p;
   uint32_t tie_before = 0, unused = 0;
-  f32_pass<ALIGNED>(P, b, rowp, pres, rep, T, m_f, invZ, 0, 0u, L, ktok, tok, tie_before);
+  f32_pass<DT, ALIGNED>(P, b, rowp, pres, rep, T, m_f, invZ, 0, 0u, L, ktok, tok, tie_before, fx);
   f32_prefix(L, 0, sh);
   const int64_t tie_tok = (int64_t)block_sum<NUC_WAVES>((uint64_t)tie_before, sh.u);
   // The first value (value desc, id asc) that the filter (rank < tk, p >= mp * max, mass ahead
@@ -1911,26 +1916,26 @@ __device__ __forceinline__ void nuc_row_f32(const KParams& P, int64_t r, F32NucL
   // The level-0 bins serve every call.
   auto descend = [&](int tk, float mp, float tp) -> bool {
     bool found = false;
-    int b0 = f32_next(L, 0, -1, true, 0u, 0ull, 0ull, T, m_f, invZ, a.backend, tk, mp, thr_minp, tp, sh);
+    int b0 = f32_next<DT>(L, 0, -1, true, 0u, 0ull, 0ull, T, m_f, invZ, a.backend, tk, mp, thr_minp, tp, fx, sh);
     // the first bin that can hold the cut, else the next non-empty one (a margin of rounding
     // may need one more)
     for (int t0 = 0; t0 < 3 && b0 >= 0 && !found; ++t0) {
       const uint64_t c0 = L.pcnt[0][b0], m0 = L.pmass[0][b0];
-      f32_pass<ALIGNED>(P, b, rowp, pres, rep, T, m_f, invZ, 1, (uint32_t)b0, L, ktok, tok, unused);
+      f32_pass<DT, ALIGNED>(P, b, rowp, pres, rep, T, m_f, invZ, 1, (uint32_t)b0, L, ktok, tok, unused, fx);
       f32_prefix(L, 1, sh);
-      int b1 = f32_next(L, 1, -1, true, (uint32_t)b0, c0, m0, T, m_f, invZ, a.backend, tk, mp, thr_minp, tp, sh);
+      int b1 = f32_next<DT>(L, 1, -1, true, (uint32_t)b0, c0, m0, T, m_f, invZ, a.backend, tk, mp, thr_minp, tp, fx, sh);
       for (int t1 = 0; t1 < 3 && b1 >= 0 && !found; ++t1) {
         const uint32_t prefix = ((uint32_t)b0 << 11) | (uint32_t)b1;
-        f32_pass<ALIGNED>(P, b, rowp, pres, rep, T, m_f, invZ, 2, prefix, L, ktok, tok, unused);
-        found = f32_walk(L, prefix, c0 + L.pcnt[1][b1], m0 + L.pmass[1][b1], T, m_f, invZ, a.backend, tk, mp,
-                         thr_minp, tp, sh);
+        f32_pass<DT, ALIGNED>(P, b, rowp, pres, rep, T, m_f, invZ, 2, prefix, L, ktok, tok, unused, fx);
+        found = f32_walk<DT>(L, prefix, c0 + L.pcnt[1][b1], m0 + L.pmass[1][b1], T, m_f, invZ, a.backend, tk, mp,
+                         thr_minp, tp, fx, sh);
         if (!found)
-          b1 = f32_next(L, 1, F32_BINS - 1 - b1, false, (uint32_t)b0, c0, m0, T, m_f, invZ, a.backend, tk, mp,
-                        thr_minp, tp, sh);
+          b1 = f32_next<DT>(L, 1, F32_BINS - 1 - b1, false, (uint32_t)b0, c0, m0, T, m_f, invZ, a.backend, tk, mp,
+                        thr_minp, tp, fx, sh);
       }
       if (!found)
-        b0 = f32_next(L, 0, F32_BINS - 1 - b0, false, 0u, 0ull, 0ull, T, m_f, invZ, a.backend, tk, mp, thr_minp,
-                      tp, sh);
+        b0 = f32_next<DT>(L, 0, F32_BINS - 1 - b0, false, 0u, 0ull, 0ull, T, m_f, invZ, a.backend, tk, mp, thr_minp,
+                      tp, fx, sh);
     }
     return found;
   };
@@ -1939,8 +1944,8 @@ __device__ __forceinline__ void nuc_row_f32(const KParams& P, int64_t r, F32NucL
     // flashinfer's min-p branch: top-p on the mass renormalised over the top-k (S_k from a
     // rank-only descent; no rank cut: the whole mass)
     const bool kf = descend(topk, 0.f, INFINITY);
-    const double Sk = kf ? sh.cut_S : (double)(L.pmass[0][0] + L.mass[0][0]) / FX_ONE;
-    top_p_eff = (float)((double)top_p * Sk);
+    const double Sk = kf ? sh.cut_S : (double)(L.pmass[0][0] + L.mass[0][0]) / fx;
+    top_p_eff = (float)((double)a.top_ps[b] * Sk);
     __syncthreads();  // (sh.cut_S read before the next descent)
   }
   const bool found = descend(topk, min_p, top_p_eff);
@@ -1969,11 +1974,11 @@ __device__ __forceinline__ void nuc_row_f32(const KParams& P, int64_t r, F32NucL
     } else {  // every value is kept
       rs.vcut = 0u;
       rs.ktie = INT_MAX;
-      rs.S_kept = (double)(L.pmass[0][0] + L.mass[0][0]) / FX_ONE;
+      rs.S_kept = (double)(L.pmass[0][0] + L.mass[0][0]) / fx;
     }
     rs.S_f = (float)rs.S_kept;
     if (count_ties) rs.flags |= FLAG_TIES_COUNTED;
-    nucleus_finish<DSV_F32>(P, r, b, s, rs, T, xt, tok, tie_tok, ro);
+    nucleus_finish<DT>(P, r, b, s, rs, T, xt, tok, tie_tok, ro);
   }
   __syncthreads();
 }
@@ -1995,7 +2000,7 @@ __global__ __launch_bounds__(NUC_THREADS) void k_nuc(KParams P) {
       nuc_row<DT, ALIGNED>(P, row, hist, sh, blockIdx.x, nullptr);
     } else {
       __shared__ F32NucShared fsh;
-      nuc_row_f32<ALIGNED>(P, row, *reinterpret_cast<F32NucLds*>(dyn), fsh, nullptr);
+      nuc_row_f32<DT, ALIGNED>(P, row, *reinterpret_cast<F32NucLds*>(dyn), fsh, nullptr);
     }
   }
 }
@@ -2090,7 +2095,7 @@ __global__ __launch_bounds__(CT, ALIGNED ? (DT == DSV_BF16 ? 7 : 6) : 5) void k_
   int topk = P.kcand;
   int64_t tok = -1;
   if (P.softmax && !P.force_greedy) {
-    if (mode != M_GREEDY) T = a.temperatures[b];
+    if (DT != DT_PROB && mode != M_GREEDY) T = a.temperatures[b];
     topk = a.top_ks[b];
     if (a.filter || a.sparse_joint) top_p = a.top_ps[b];
     if (pen) {
@@ -2223,7 +2228,16 @@ __global__ __launch_bounds__(CT, ALIGNED ? (DT == DSV_BF16 ? 7 : 6) : 5) void k_
   out.pad = 0;
 
   // the softmax partial sum (support-list rows of the step only when their top-p test needs Z)
-  if (P.softmax && mode != M_GREEDY && cbest && (mode != M_LIST || list_needs_z(a, top_p))) {
+  if constexpr (DT == DT_PROB) {  // the chunk's mass, in float64 (values past the row: -inf)
+    double st_ = 0.0;
+#pragma unroll
+    for (int u = 0; u < CV; ++u) {
+#pragma unroll
+      for (int e = 0; e < n; ++e) st_ += (double)fmaxf(vec_elem<DT>(v[u], e), 0.f);
+    }
+    out.s = block_sum<CT / WAVE>(st_, sd);
+    reg_fence(v);
+  } else if (P.softmax && mode != M_GREEDY && cbest && (mode != M_LIST || list_needs_z(a, top_p))) {
     const float c2 = log2e_over(T);
     const float mc2 = out.m * c2;
     float st_ = 0.f;
@@ -2392,7 +2406,7 @@ __global__ __launch_bounds__(CT, ALIGNED ? (DT == DSV_BF16 ? 7 : 6) : 5) void k_
           hit = ((int)d.x > (int)d.y ? (int)d.x : (int)d.y) >= t0;
         } else if (pos_thr) {
           hit = max(max((int)v[u].x, (int)v[u].y), max((int)v[u].z, (int)v[u].w)) >= t0;
-        } else if constexpr (DT == DSV_F32) {
+        } else if constexpr (DT != DSV_BF16) {
           // float bits as signed integers with the negative values' magnitude bits flipped
           // order as their keys do (key = image ^ 2^31), -0 one below +0; a zero bound (the key
           // of +-0) is lowered by one to take -0 in
@@ -2589,7 +2603,7 @@ __device__ __forceinline__ void defer_nucleus(const KParams& P, int64_t r, float
   int32_t arg = readlane_at(arg_l, at_max ? __ffsll((long long)at_max) - 1 : 0);
   if (arg == INT_MAX) arg = 0;
   const float c2 = log2e_over(T);
-  const double Z = wave_sum(m_l > -INFINITY ? s_l * (double)__builtin_amdgcn_exp2f((m_l - M) * c2) : 0.0);
+  const double Z = DT == DT_PROB ? wave_sum(s_l) : wave_sum(m_l > -INFINITY ? s_l * (double)__builtin_amdgcn_exp2f((m_l - M) * c2) : 0.0);
   RowSum rs;
   rs.mode = M_HIST;
   rs.argmax = arg;
@@ -2600,7 +2614,7 @@ __device__ __forceinline__ void defer_nucleus(const KParams& P, int64_t r, float
   rs.flags = FLAG_FULL_HIST;
   rs.norm = 0;
   rs.m_f = M / T;
-  rs.invZ = (float)(1.0 / Z);
+  rs.invZ = DT == DT_PROB ? 1.f : (float)(1.0 / Z);
   rs.Z = Z;
   rs.S_kept = 1.0;
   rs.S_f = 1.f;
@@ -2761,8 +2775,8 @@ __global__ __launch_bounds__(CT, 4) void k_merge(KParams P) {
     }
     return;
   }
-  const int mode = row_mode(a, b, 0);
-  const float T = a.temperatures[b];
+  int mode = row_mode(a, b, 0);
+  const float T = DT == DT_PROB ? 1.f : a.temperatures[b];
   const int cap = req_cap(a, b);
   const bool resid = s < cap - 1;  // the row tests draft s+1, and ends the prefix when it is rejected
   const bool tests = a.candidates != nullptr && resid;
@@ -2795,6 +2809,14 @@ __global__ __launch_bounds__(CT, 4) void k_merge(KParams P) {
   if (tid >= WAVE && tid < 2 * WAVE)
     fetch_q_wave<DT>(P, b, s, tests, row_ptr(a, r), mode == M_UNF || mode == M_HIST, ds, ql);
   __syncthreads();
+  if constexpr (DT == DT_PROB) {
+    // a top-p of 1 or more cuts a row whose raw mass is above it
+    if (mode == M_UNF && P.top_p_raw) {
+      double mass = 0.0;
+      for (int c = 0; c < P.C; ++c) mass += pre.cs[c].s;
+      if ((a.backend == DSV_BACKEND_PYTORCH ? (double)(float)mass : mass) > (double)pre.top_p) mode = M_HIST;
+    }
+  }
   if (mode == M_HIST) {
     if constexpr (DT == DSV_BF16)
       merge_nucleus<DT>(P, r, b, s, T, ns, ds, pre, &ro);
@@ -2976,7 +2998,7 @@ __global__ __launch_bounds__(FCT) void k_final(KParams P) {
         nuc_row<DT, ALIGNED>(P, r, reinterpret_cast<uint32_t*>(dyn), nsh, b, &fro);
       } else {
         __shared__ F32NucShared fsh;
-        nuc_row_f32<ALIGNED>(P, r, *reinterpret_cast<F32NucLds*>(dyn), fsh, &fro);
+        nuc_row_f32<DT, ALIGNED>(P, r, *reinterpret_cast<F32NucLds*>(dyn), fsh, &fro);
       }
       __syncthreads();
       if (acc < cap - 1 && fro.ok) {
@@ -3111,13 +3133,11 @@ __device__ __forceinline__ void dense_p_spans(const KParams& P, int64_t r, int c
         for (int e = 0; e < n; ++e)
           if ((int64_t)lst[e].id == j) {
             v = lst[e].P;
-            if (P.raw_p && P.src_p) {  // the input probability itself
-              v = P.src_p[r * P.src_stride + j];
-            } else if (P.raw_p) {  // the unrenormalised p: recomputed from the adjusted logit
+            if (P.raw_p) {  // the unrenormalised p: recomputed from the adjusted logit
               float x = load_elem<DT>(row_ptr(a, r), j);
               if (P.pbits && pen_test(P, b, j))
                 x = penalize<DT>(x, a.presence ? a.presence[b] : 0.f, a.repetition ? a.repetition[b] : 1.f);
-              v = prob_of(x, a.temperatures[b], rs.m_f, rs.invZ);
+              v = weight_of<DT>(x, DT == DT_PROB ? 1.f : a.temperatures[b], rs.m_f, rs.invZ);
             }
           }
       if (vec_ok) put(i, v); else put1(i, v);
@@ -3127,7 +3147,7 @@ __device__ __forceinline__ void dense_p_spans(const KParams& P, int64_t r, int c
   const bool pen = P.pbits != nullptr;
   const float pres = pen && a.presence ? a.presence[b] : 0.f;
   const float rep = pen && a.repetition ? a.repetition[b] : 1.f;
-  const float T = a.temperatures[b];
+  const float T = DT == DT_PROB ? 1.f : a.temperatures[b];
   const char* rowp = row_ptr(a, r);
   const bool hist = mode == M_HIST;
   int32_t tbefore = 0;
@@ -3165,9 +3185,7 @@ __device__ __forceinline__ void dense_p_spans(const KParams& P, int64_t r, int c
     const uint32_t k = key_of<DT>(x);
     const bool kept = !hist || k > rs.vcut || (k == rs.vcut && (int64_t)tbefore + seen < (int64_t)rs.ktie);
     if (kept)
-      v = P.raw_p ? (P.src_p ? (jlo + i < V ? P.src_p[r * P.src_stride + jlo + i] : 0.f)  // (ids past the row: -inf)
-                             : prob_of(x, T, rs.m_f, rs.invZ))
-                  : (float)dense_P(rs, T, x);
+      v = P.raw_p ? weight_of<DT>(x, T, rs.m_f, rs.invZ) : (float)dense_P<DT>(rs, T, x);
     seen += hist && k == rs.vcut;
     if (vec_ok) put(i, v); else put1(i, v);
   });
@@ -3271,13 +3289,11 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
             for (int q = 0; q < nl; ++q)
               if ((int64_t)lst[q].id == j) {
                 x[e] = lst[q].P;
-                if (P.raw_p && P.src_p) {  // the input probability itself
-                  x[e] = P.src_p[r * P.src_stride + j];
-                } else if (P.raw_p) {  // the unrenormalised p: recomputed from the adjusted logit
+                if (P.raw_p) {  // the unrenormalised p: recomputed from the adjusted logit
                   float xv = load_elem<DT>(row_ptr(a, r), j);
                   if (P.pbits && pen_test(P, b, j))
                     xv = penalize<DT>(xv, a.presence ? a.presence[b] : 0.f, a.repetition ? a.repetition[b] : 1.f);
-                  x[e] = prob_of(xv, a.temperatures[b], rs.m_f, rs.invZ);
+                  x[e] = weight_of<DT>(xv, DT == DT_PROB ? 1.f : a.temperatures[b], rs.m_f, rs.invZ);
                 }
               }
           }
@@ -3297,7 +3313,7 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
   const bool pen = P.pbits != nullptr;
   const float pres = pen && a.presence ? a.presence[b] : 0.f;
   const float rep = pen && a.repetition ? a.repetition[b] : 1.f;
-  const float T = a.temperatures[b];
+  const float T = DT == DT_PROB ? 1.f : a.temperatures[b];
   const char* rowp = row_ptr(a, r);
   uint4 v[CV];
   const int64_t nfull = hi / n;
@@ -3387,91 +3403,16 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
         const bool tie = hist && k == rs.vcut;
         const bool kept = !hist || k > rs.vcut || (tie && (int64_t)rank0[u] + seen < (int64_t)rs.ktie);
         seen += tie ? 1 : 0;
-        const float pe = prob_of(xe, T, rs.m_f, rs.invZ);
+        const float pe = weight_of<DT>(xe, T, rs.m_f, rs.invZ);
         x[e] = kept ? (DIV ? pe / rs.S_f : pe) : 0.f;
       }
       store_vec(j0, x);
     }
   };
-  // raw_p with the input probabilities (logs as the rows): the kept entries copied from them
-  auto copy_rows = [&]() {
-    const float* srow = P.src_p + r * P.src_stride;
-#pragma unroll
-    for (int u = 0; u < CV; ++u) {
-      const int64_t j0 = (v0 + (int64_t)u * CT + tid) * n;
-      if (j0 >= hi) continue;
-      float x[n];
-      int32_t seen = 0;
-#pragma unroll
-      for (int e = 0; e < n; ++e) {
-        const uint32_t k = key_of<DT>(vec_elem<DT>(v[u], e));
-        const bool tie = hist && k == rs.vcut;
-        const bool kept = !hist || k > rs.vcut || (tie && (int64_t)rank0[u] + seen < (int64_t)rs.ktie);
-        seen += tie ? 1 : 0;
-        x[e] = kept && j0 + e < hi ? srow[j0 + e] : 0.f;
-      }
-      store_vec(j0, x);
-    }
-  };
-  if (P.raw_p && P.src_p)
-    copy_rows();
-  else if (!P.raw_p && (rs.mode == M_HIST || rs.norm))
+  if (!P.raw_p && (rs.mode == M_HIST || rs.norm))
     write_rows(std::true_type{});
   else
     write_rows(std::false_type{});
-}
-
-// ---------------------------------------------------------------------------------------
-// filter_target_probs on probabilities (runtime/worker.py:473-508): each row becomes a request
-// of its own at temperature 1 whose logits are log p (softmax(log p) = p / sum(p), and top-k,
-// min-p and the order of the values are those of p).  One workgroup per row writes log p and
-// the row's float64 mass, and the row's parameters from its request's: the top-p divided by the
-// mass when the backend compares the raw mass ranked ahead with top_p (top_p_over_mass).
-// ---------------------------------------------------------------------------------------
-__global__ __launch_bounds__(CT) void k_prob_prep(const float* __restrict__ probs, int64_t pstride, int64_t V,
-                                                  int32_t T, const int32_t* top_ks, const float* top_ps,
-                                                  const float* min_ps, int32_t top_p_over_mass, int32_t vec4,
-                                                  float* __restrict__ logs, int64_t lstride, int32_t* row_k,
-                                                  float* row_p, float* row_minp, float* row_t) {
-  __shared__ double sd[CT / WAVE];
-  const int64_t r = blockIdx.x;
-  const float* prow = probs + r * pstride;
-  float* lrow = logs + r * lstride;
-  double mass = 0.0;
-  if (vec4) {  // rows 16-byte aligned, V a multiple of 4: four 16-byte loads in flight a thread
-    constexpr int U = 4;
-    const int64_t nv = V / 4;
-    for (int64_t q0 = threadIdx.x; q0 < nv; q0 += (int64_t)CT * U) {
-      float4 p[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t q = q0 + (int64_t)u * CT;
-        p[u] = q < nv ? reinterpret_cast<const float4*>(prow)[q] : make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t q = q0 + (int64_t)u * CT;
-        if (q >= nv) continue;
-        mass += (double)p[u].x + (double)p[u].y + (double)p[u].z + (double)p[u].w;
-        reinterpret_cast<float4*>(lrow)[q] = make_float4(logf(p[u].x), logf(p[u].y), logf(p[u].z), logf(p[u].w));
-      }
-    }
-  } else {
-    for (int64_t j = threadIdx.x; j < V; j += CT) {
-      const float p = prow[j];
-      mass += (double)p;
-      lrow[j] = logf(p);
-    }
-  }
-  mass = block_sum<CT / WAVE>(mass, sd);
-  if (threadIdx.x == 0) {
-    const int64_t b = r / T;
-    const float tp = top_ps ? top_ps[b] : 1.f;
-    row_k[r] = top_ks[b];
-    row_p[r] = top_p_over_mass && mass > 0.0 ? (float)((double)tp / mass) : tp;
-    row_minp[r] = min_ps ? min_ps[b] : 0.f;
-    row_t[r] = 1.f;
-  }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -3586,18 +3527,29 @@ static int64_t align_up(int64_t x, int64_t al) { return (x + al - 1) / al * al; 
 struct WsLayout {
   int64_t rowsum, lists, cstat, cand, hpart, nhist, nuc, rbonus, rties, plans, step_ok, req_cnt, deferred, pbits, total;
 };
+// f(row type) with the type as a constant: DSV_BF16, DSV_F32 or DT_PROB.
+template <int DT>
+struct RowType {
+  static constexpr int value = DT;
+};
+template <class F>
+static void for_row_type(int dtype, int prob, F&& f) {
+  if (prob)
+    f(RowType<DT_PROB>{});
+  else if (dtype == DSV_BF16)
+    f(RowType<DSV_BF16>{});
+  else
+    f(RowType<DSV_F32>{});
+}
+
 static void launch_chunk(const KParams& P, int dtype, unsigned grid, hipStream_t stream) {
-  if (dtype == DSV_BF16) {
+  for_row_type(dtype, P.prob, [&](auto t) {
+    constexpr int DT = decltype(t)::value;
     if (P.aligned)
-      hipLaunchKernelGGL((k_chunk<DSV_BF16, true>), dim3(grid), dim3(CT), 0, stream, P);
+      hipLaunchKernelGGL((k_chunk<DT, true>), dim3(grid), dim3(CT), 0, stream, P);
     else
-      hipLaunchKernelGGL((k_chunk<DSV_BF16, false>), dim3(grid), dim3(CT), 0, stream, P);
-  } else {
-    if (P.aligned)
-      hipLaunchKernelGGL((k_chunk<DSV_F32, true>), dim3(grid), dim3(CT), 0, stream, P);
-    else
-      hipLaunchKernelGGL((k_chunk<DSV_F32, false>), dim3(grid), dim3(CT), 0, stream, P);
-  }
+      hipLaunchKernelGGL((k_chunk<DT, false>), dim3(grid), dim3(CT), 0, stream, P);
+  });
 }
 
 static int chunks_per_row(int64_t vocab, int dtype) {
@@ -3728,45 +3680,30 @@ static int launch_rows(const KParams& P, bool hist_possible, bool profile, hipSt
   launch_chunk(P, a.logits_dtype, (unsigned)(a.rows * P.C), stream);
   if (profile && g_prof_start && g_prof_stop && hipEventRecord(g_prof_stop, stream) != hipSuccess)
     DSV_FAIL(DSV_ERR_LAUNCH, "dsv_verify: cannot record the profiling stop event");
-  if (a.logits_dtype == DSV_BF16) {
+  for_row_type(a.logits_dtype, P.prob, [&](auto t) {
+    constexpr int DT = decltype(t)::value;
     if (P.aligned)
-      hipLaunchKernelGGL((k_merge<DSV_BF16, true>), dim3((unsigned)a.rows), dim3(CT), 0, stream, P);
+      hipLaunchKernelGGL((k_merge<DT, true>), dim3((unsigned)a.rows), dim3(CT), 0, stream, P);
     else
-      hipLaunchKernelGGL((k_merge<DSV_BF16, false>), dim3((unsigned)a.rows), dim3(CT), 0, stream, P);
-  } else {
-    if (P.aligned)
-      hipLaunchKernelGGL((k_merge<DSV_F32, true>), dim3((unsigned)a.rows), dim3(CT), 0, stream, P);
-    else
-      hipLaunchKernelGGL((k_merge<DSV_F32, false>), dim3((unsigned)a.rows), dim3(CT), 0, stream, P);
-  }
+      hipLaunchKernelGGL((k_merge<DT, false>), dim3((unsigned)a.rows), dim3(CT), 0, stream, P);
+  });
   DSV_CHECK_LAUNCH("k_chunk / k_merge");
   if (hist_possible && !P.final_nuc) {  // rows the merge listed: the full histogram (bf16) or radix descent (fp32)
     // (bf16 workgroups each own a global histogram area; fp32 ones work in LDS alone, one per CU)
     const int cap = a.logits_dtype == DSV_BF16 ? NUC_GRID : NUC_GRID_F32;
     const int grid = (int)(a.rows < cap ? a.rows : cap);
-    if (a.logits_dtype == DSV_BF16) {
-      const size_t nuc_lds = (size_t)HIST_WORDS * 4;
-      if (P.aligned) {
-        (void)hipFuncSetAttribute((const void*)k_nuc<DSV_BF16, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)nuc_lds);
-        hipLaunchKernelGGL((k_nuc<DSV_BF16, true>), dim3(grid), dim3(NUC_THREADS), nuc_lds, stream, P);
-      } else {
-        (void)hipFuncSetAttribute((const void*)k_nuc<DSV_BF16, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)nuc_lds);
-        hipLaunchKernelGGL((k_nuc<DSV_BF16, false>), dim3(grid), dim3(NUC_THREADS), nuc_lds, stream, P);
-      }
-    } else {
-      const size_t nuc_lds = sizeof(F32NucLds);
-      if (P.aligned) {
-        (void)hipFuncSetAttribute((const void*)k_nuc<DSV_F32, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)nuc_lds);
-        hipLaunchKernelGGL((k_nuc<DSV_F32, true>), dim3(grid), dim3(NUC_THREADS), nuc_lds, stream, P);
-      } else {
-        (void)hipFuncSetAttribute((const void*)k_nuc<DSV_F32, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)nuc_lds);
-        hipLaunchKernelGGL((k_nuc<DSV_F32, false>), dim3(grid), dim3(NUC_THREADS), nuc_lds, stream, P);
-      }
-    }
+    for_row_type(a.logits_dtype, P.prob, [&](auto t) {
+      constexpr int DT = decltype(t)::value;
+      const size_t nuc_lds = DT == DSV_BF16 ? (size_t)HIST_WORDS * 4 : sizeof(F32NucLds);
+      auto go = [&](auto kernel) {
+        (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)nuc_lds);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(NUC_THREADS), nuc_lds, stream, P);
+      };
+      if (P.aligned)
+        go(k_nuc<DT, true>);
+      else
+        go(k_nuc<DT, false>);
+    });
     DSV_CHECK_LAUNCH("k_nuc");
   }
   return DSV_OK;
@@ -3825,17 +3762,13 @@ static int launch_target(KParams& P, bool hist_possible, float* out, int64_t out
   const int rc = launch_rows(P, hist_possible, false, stream);
   if (rc != DSV_OK) return rc;
   const dim3 grid((unsigned)(a.rows * P.C));
-  if (a.logits_dtype == DSV_BF16) {
+  for_row_type(a.logits_dtype, P.prob, [&](auto t) {
+    constexpr int DT = decltype(t)::value;
     if (P.aligned)
-      hipLaunchKernelGGL((k_dense_p<DSV_BF16, true>), grid, dim3(CT), 0, stream, P, out, out_stride);
+      hipLaunchKernelGGL((k_dense_p<DT, true>), grid, dim3(CT), 0, stream, P, out, out_stride);
     else
-      hipLaunchKernelGGL((k_dense_p<DSV_BF16, false>), grid, dim3(CT), 0, stream, P, out, out_stride);
-  } else {
-    if (P.aligned)
-      hipLaunchKernelGGL((k_dense_p<DSV_F32, true>), grid, dim3(CT), 0, stream, P, out, out_stride);
-    else
-      hipLaunchKernelGGL((k_dense_p<DSV_F32, false>), grid, dim3(CT), 0, stream, P, out, out_stride);
-  }
+      hipLaunchKernelGGL((k_dense_p<DT, false>), grid, dim3(CT), 0, stream, P, out, out_stride);
+  });
   DSV_CHECK_LAUNCH("k_dense_p");
   return DSV_OK;
 }
@@ -3856,15 +3789,20 @@ extern "C" int dsv_target_probs(const dsv_verify_args* args, float* out, int64_t
   return launch_target(P, hist_possible, out, out_stride, stream);
 }
 
-// the log rows' stride (floats), and the layout of the filter workspace: log p, the rows'
-// parameters, then the row kernels' workspace with each row a request of its own
-static int64_t filter_log_stride(int64_t vocab) { return align_up(vocab, 64); }
-static int64_t filter_head_bytes(int64_t rows, int64_t vocab) {
-  return align_up(rows * filter_log_stride(vocab) * 4, 256) + 4 * align_up(rows * 4, 256);
+// filter_target_probs on probabilities (runtime/worker.py:473-508): the row kernels on the given rows
+// as they are (DT_PROB: a value's weight is the value), one read of each row where it needs no cut,
+// masses and top-p in the rows' own units.  A pass that wrote each row's logarithms for the softmax
+// kernels to take (and their exponentials) made it 553 us at 32 x 17 rows of 151936, this 331, and
+// 1.7e-7 off float64, this 1.8e-8.
+__global__ void k_fill_ones(float* out, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = 1.f;
 }
+
 extern "C" int64_t dsv_filter_workspace_bytes(int64_t rows, int64_t vocab) {
   if (rows < 0 || vocab < 1) return -1;
-  return filter_head_bytes(rows, vocab) + dsv_verify_workspace_bytes(rows, (int32_t)(rows > 0 ? rows : 1), 1, vocab);
+  const int64_t n = rows > 0 ? rows : 1;  // (at most a request a row; their top-p where none is given)
+  return align_up(n * 4, 256) + dsv_verify_workspace_bytes(rows, (int32_t)n, 1, vocab);
 }
 
 extern "C" int dsv_filter_probs(const dsv_verify_args* args, const float* probs, int64_t probs_stride, float* out,
@@ -3886,32 +3824,16 @@ extern "C" int dsv_filter_probs(const dsv_verify_args* args, const float* probs,
   if (a.workspace_bytes < need)
     DSV_FAIL(DSV_ERR_WORKSPACE, "dsv_filter_probs: workspace %lld < %lld bytes", (long long)a.workspace_bytes,
              (long long)need);
-  const int64_t rows = a.rows, lstride = filter_log_stride(a.vocab);
-  char* ws = reinterpret_cast<char*>(a.workspace);
-  float* logs = reinterpret_cast<float*>(ws);
-  char* prm = ws + align_up(rows * lstride * 4, 256);
-  const int64_t pb = align_up(rows * 4, 256);
-  int32_t* row_k = reinterpret_cast<int32_t*>(prm);
-  float* row_p = reinterpret_cast<float*>(prm + pb);
-  float* row_minp = reinterpret_cast<float*>(prm + 2 * pb);
-  float* row_t = reinterpret_cast<float*>(prm + 3 * pb);
-  const int32_t vec4 = (uintptr_t)probs % 16 == 0 && probs_stride % 4 == 0 && a.vocab % 4 == 0;
-  hipLaunchKernelGGL(k_prob_prep, dim3((unsigned)rows), dim3(CT), 0, stream, probs, probs_stride, a.vocab, a.T,
-                     a.top_ks, a.top_ps, a.min_ps, top_p_over_mass, vec4, logs, lstride, row_k, row_p, row_minp,
-                     row_t);
-  DSV_CHECK_LAUNCH("k_prob_prep");
-  // each row a request at temperature 1, no penalties, no drafts
+  const int64_t head = align_up(a.rows * 4, 256);
+  float* ones = reinterpret_cast<float*>(a.workspace);
+  // every row filtered, none greedy, no penalties, no drafts
   dsv_verify_args r = a;
-  r.logits = logs;
+  r.logits = probs;
   r.logits_dtype = DSV_F32;
-  r.row_stride = lstride;
-  r.bs = (int32_t)rows;
-  r.T = 1;
-  r.verify_lens = nullptr;  // every row is filtered
-  r.temperatures = row_t;
-  r.top_ks = row_k;
-  r.top_ps = row_p;
-  r.min_ps = a.min_ps ? row_minp : nullptr;
+  r.row_stride = probs_stride;
+  r.verify_lens = nullptr;
+  r.temperatures = ones;  // (not read)
+  if (!a.top_ps) r.top_ps = ones;
   r.any_greedy = 0;
   r.sparse_joint = 0;
   r.hist_ids = nullptr;
@@ -3919,15 +3841,19 @@ extern "C" int dsv_filter_probs(const dsv_verify_args* args, const float* probs,
   r.presence = nullptr;
   r.repetition = nullptr;
   r.candidates = nullptr;
-  r.workspace = ws + filter_head_bytes(rows, a.vocab);
-  r.workspace_bytes = a.workspace_bytes - filter_head_bytes(rows, a.vocab);
+  r.workspace = reinterpret_cast<char*>(a.workspace) + head;
+  r.workspace_bytes = a.workspace_bytes - head;
   KParams P;
   bool hist_possible = false;
   const int rc = verify_prepare(r, false, "dsv_filter_probs", P, hist_possible);
   if (rc != DSV_OK) return rc;
+  P.prob = 1;
   P.raw_p = normalize ? 0 : 1;
-  P.src_p = normalize ? nullptr : probs;
-  P.src_stride = probs_stride;
+  P.top_p_raw = top_p_over_mass ? 1 : 0;
+  if (!a.top_ps) {
+    hipLaunchKernelGGL(k_fill_ones, dim3((unsigned)((a.bs + 255) / 256)), dim3(256), 0, stream, ones, a.bs);
+    DSV_CHECK_LAUNCH("k_fill_ones");
+  }
   return launch_target(P, hist_possible, out, out_stride, stream);
 }
 

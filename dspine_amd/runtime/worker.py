@@ -59,13 +59,10 @@ def filter_target_probs(probs, sampling_info, t, bs, sampling_backend, normalize
     """runtime/worker.py:473-508 on given probabilities [bs*t, V]: the backend filter, then
     (``normalize``) renormalised; without a filter flag the input is returned as a view.
 
-    One library call (``dsv_filter_probs``): a pre-pass writes log p and each row's float64
-    mass, then the HIP row kernels filter every row as a request of its own at temperature 1
-    (softmax(log p) = p / sum(p), which renormalises to the same distribution; top-k and min-p,
-    a ratio to the row's top p, select the same ids).  The reference's top-p test compares the
-    raw mass ranked ahead of an id with top_p (:52-67; flashinfer's joint branch likewise, its
-    min-p branch renormalises over the top-k first), so those rows' top_p is divided by the
-    row's mass.  With ``normalize`` False the kept entries are the input values themselves."""
+    One library call (``dsv_filter_probs``): the HIP row kernels on the probabilities as they
+    are.  The reference's top-p test compares the raw mass ranked ahead of an id with top_p
+    (:52-67; flashinfer's joint branch likewise; its min-p branch renormalises over the top-k
+    first).  With ``normalize`` False the kept entries are the input values themselves."""
     need_k = bool(getattr(sampling_info, "need_top_k_sampling", False))
     need_p = bool(getattr(sampling_info, "need_top_p_sampling", False))
     need_min_p = bool(getattr(sampling_info, "need_min_p_sampling", False))

@@ -223,14 +223,13 @@ int dsv_target_probs(const dsv_verify_args* args, float* out, int64_t out_stride
 
 /* The backend filter on given probabilities probs [rows, vocab] float32 (row stride           */
 /* probs_stride; runtime/worker.py:473-508 filter_target_probs), rows = bs * T, the sampling   */
-/* parameters per request as in dsv_verify_args (temperatures and the history are ignored:   */
-/* each row is filtered at temperature 1, none is greedy).  out [rows, vocab]: the kept      */
-/* entries renormalised (normalize = 0: the input values themselves), zeros elsewhere.        */
-/* top_p_over_mass = 1 compares the raw mass ranked ahead of an entry with top_p (the         */
-/* pytorch backend, flashinfer's joint branch): each row's top_p is divided by its float64    */
-/* mass.  Requires a filter flag and rows <= 65535; the workspace holds                       */
-/* dsv_filter_workspace_bytes(rows, vocab) bytes.  Entries that round to the same log p tie   */
-/* (broken by the lower id).                                                                  */
+/* parameters per request as in dsv_verify_args (temperatures and the history are ignored,   */
+/* no row is greedy; top_ps NULL: 1).  The values are taken as they are, in the row's own units: */
+/* out [rows, vocab]: the kept entries over their mass (normalize = 0: the input values        */
+/* themselves), zeros elsewhere.  top_p_over_mass = 1 compares the raw mass ranked ahead of an  */
+/* entry with top_p (the pytorch backend, flashinfer's joint branch), 0 its share of the row's  */
+/* mass.  Requires a filter flag and rows <= 65535; the workspace holds                         */
+/* dsv_filter_workspace_bytes(rows, vocab) bytes.                                               */
 int64_t dsv_filter_workspace_bytes(int64_t rows, int64_t vocab);
 int dsv_filter_probs(const dsv_verify_args* args, const float* probs, int64_t probs_stride, float* out,
                      int64_t out_stride, int32_t normalize, int32_t top_p_over_mass, dsv_stream_t stream);

@@ -416,6 +416,43 @@ def test_filter_target_probs_unnormalised_rows(device, backend, min_p):
         assert not torch.equal(unit > 0, ref > 0)
 
 
+@pytest.mark.parametrize("V", [5, 997, 12289, 24580])
+@pytest.mark.parametrize("backend,min_p", [("pytorch", 0.0), ("pytorch", 0.04), ("flashinfer", 0.0),
+                                           ("flashinfer", 0.04)])
+def test_filter_target_probs_row_forms(device, V, backend, min_p):
+    """Rows of any mass (2^-30 to 3000, zeros in them, one a single value, one of mass just over a
+    top-p of 1), every kind of cut (top-k alone, top-p alone, both, none), at the edges of the chunks,
+    against the oracle on the same rows: kept values bit for bit, renormalised ones to a rounding of
+    the mass."""
+    from dspine_amd.runtime.worker import filter_target_probs
+
+    O = _O()
+    g = torch.Generator().manual_seed(V)
+    ks = torch.tensor([0, 0, 20, 20, 0, 70, 1, 0])
+    ps = torch.tensor([0.9, 1.0, 1.0, 0.8, 0.5, 0.95, 1.0, 0.3])
+    bs, T = len(ks), 2
+    p = torch.softmax(torch.randn(bs * T, V, generator=g) * 2.0, -1)
+    p[::3, V // 2:] = 0
+    p = p / p.sum(-1, keepdim=True)
+    p[3] = 0
+    p[3, V - 1] = 0.25
+    p[[4, 9]] *= 2.0 ** -30
+    p[2] *= 1.0 + 2.0 ** -10
+    if backend == "pytorch":  # (raw top-p: a large mass keeps its first values)
+        p[[8, 11]] *= 3000.0
+    info = W.sampling_info(torch.ones(bs), ks, ps, torch.full((bs,), min_p))
+    info.is_any_greedy = False
+    for normalize in (True, False):
+        got = filter_target_probs(p.to(device), W.info_to(info, device), T, bs, backend, normalize).cpu()
+        # (in float64: the oracle's float32 prefix sums would decide the last ranks of a wide row)
+        ref = O.filter_target_probs(p.double() if backend == "flashinfer" else p, info, T, bs, backend, normalize)
+        assert torch.equal(got > 0, ref > 0)
+        if normalize:
+            torch.testing.assert_close(got.double(), ref.double(), rtol=1e-6, atol=0)
+        else:
+            assert torch.equal(got.double(), ref.double())
+
+
 def test_softmax_temp(device):
     from dspine_amd.runtime.worker import SoftmaxTemp
 
