@@ -402,7 +402,7 @@ __device__ __forceinline__ void span_load(const KParams& P, int b, const char* r
       if (jlo + u * n + n > chi) sp.v[u] = load_vec<DT>(rowp, jlo / n + u, chi, false);
   } else {
 #pragma unroll
-    for (int u = 0; u < SV; ++u) sp.v[u] = load_vec<DT>(rowp, jlo / n + u, chi, false);
+    for (int u = 0; u < SV; ++u) sp.v[u] = load_vec_any<DT>(rowp, jlo / n + u, chi);
   }
   sp.blo = 0;
   sp.bhi = 0;
@@ -1736,7 +1736,7 @@ __device__ __forceinline__ void f32_pass(const KParams& P, int b, const char* ro
       if constexpr (ALIGNED)
         w[u] = load_vec_raw(rowp, vi < ve ? vi : ve - 1);
       else
-        w[u] = load_vec<DSV_F32>(rowp, vi, V, false);
+        w[u] = load_vec_any<DSV_F32>(rowp, vi, V);
       const uint32_t bw = pen ? pen_bits(P, b, (vi < ve ? vi : 0) * 4, 4) : 0u;
       bits[u] = vi < ve ? bw : 0u;
     }
@@ -2061,7 +2061,7 @@ __global__ __launch_bounds__(CT, ALIGNED ? (DT == DSV_BF16 ? 7 : 6) : 5) void k_
     for (int u = 0; u < CV; ++u) v[u] = buf_load16(rs, (uint32_t)tid * 16u, (uint32_t)(u * CT * 16));
   } else {
 #pragma unroll
-    for (int u = 0; u < CV; ++u) v[u] = load_vec<DT>(rowp, v0 + (int64_t)u * CT + tid, hi, false);
+    for (int u = 0; u < CV; ++u) v[u] = load_vec_any<DT>(rowp, v0 + (int64_t)u * CT + tid, hi);
   }
   if (hist_ahead) {
     for (int i = tid; i < CHE / 32; i += CT) s_pb[i] = 0u;
@@ -3081,7 +3081,7 @@ __global__ __launch_bounds__(FCT) void k_final(KParams P) {
 // The target distribution of one (row, chunk) written out densely with each thread a span of
 // consecutive ids (runtime/worker.py:440-508): the ordered path of k_dense_p -- rows whose cut
 // keeps only some of the values at the cut key (their rank in id order decides), and outputs
-// that are not 16-byte aligned.
+// that are not 4-byte aligned.
 // ---------------------------------------------------------------------------------------
 template <int DT, bool ALIGNED>
 __device__ __forceinline__ void dense_p_spans(const KParams& P, int64_t r, int c, int b, const RowSum& rs, int mode,
@@ -3223,9 +3223,9 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
   const RowSum rs = P.rowsum[r];
   const int mode = live_row ? rs.mode : M_SKIP;
   const bool hist = mode == M_HIST;
-  const bool vec_ok = (out_stride % 4 == 0) && ((uintptr_t)out % 16 == 0);
   // a cut that keeps only the first ktie values of the cut key in id order (partial ties)
   const bool part_ties = hist && rs.ktie > 0 && rs.ktie != INT_MAX;
+  const bool vec_ok = (out_stride % 4 == 0 || (uintptr_t)orow % 4 == 0);  // (any row of floats)
   if (!vec_ok || (part_ties && (rs.flags & FLAG_FULL_HIST) && !(rs.flags & FLAG_TIES_COUNTED))) {
     dense_p_spans<DT, ALIGNED>(P, r, c, b, rs, mode, out, out_stride);
     return;
@@ -3238,7 +3238,7 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
     if (j0 + n <= hi) {
 #pragma unroll
       for (int q = 0; q < n / 4; ++q)
-        *reinterpret_cast<float4*>(orow + j0 + 4 * q) = make_float4(x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]);
+        *reinterpret_cast<v4f4_t*>(orow + j0 + 4 * q) = v4f_t{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
     } else {
 #pragma unroll
       for (int e = 0; e < n; ++e)
@@ -3300,7 +3300,7 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
         }
       }
       if (j0 + G <= hi) {
-        *reinterpret_cast<float4*>(orow + j0) = make_float4(x[0], x[1], x[2], x[3]);
+        *reinterpret_cast<v4f4_t*>(orow + j0) = v4f_t{x[0], x[1], x[2], x[3]};
       } else {
 #pragma unroll
         for (int e = 0; e < G; ++e)
@@ -3329,7 +3329,7 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
     }
   } else {
 #pragma unroll
-    for (int u = 0; u < CV; ++u) v[u] = load_vec<DT>(rowp, v0 + (int64_t)u * CT + tid, hi, false);
+    for (int u = 0; u < CV; ++u) v[u] = load_vec_any<DT>(rowp, v0 + (int64_t)u * CT + tid, hi);
   }
   if (pen) {
     for (int i = tid; i < CHE / 32; i += CT) {

@@ -353,6 +353,40 @@ def test_verify_row_layouts(device, dtype, V, stride):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("offset,V,stride", [(1, 20483, 20483), (3, 12289, 12291), (2, 997, 999), (7, 41003, 41006)])
+def test_rows_of_any_alignment(device, dtype, offset, V, stride):
+    """Rows that start at any element (an odd vocabulary, a view into a larger buffer), P written to rows
+    of an odd stride: the same bits as rows copied to 16-byte boundaries."""
+    from dspine_amd.kernels.dspine import topk
+    from dspine_amd.verification.caps import accept_greedy
+    from dspine_amd.verify import target_probs
+
+    g = torch.Generator().manual_seed(V)
+    bs, T = 4, 3
+    x = (torch.randn(bs * T, V, generator=g) * 2.5).to(dtype)
+    buf = torch.full((bs * T * stride + 16,), float("nan"), dtype=dtype, device=device)
+    odd = buf[offset:].as_strided((bs * T, V), (stride, 1))
+    odd.copy_(x)
+    pad = torch.zeros(bs * T, (V + 63) // 64 * 64, dtype=dtype, device=device)[:, :V]
+    pad.copy_(x)
+    for a, b in zip(topk(odd, 20), topk(pad, 20)):
+        assert torch.equal(a, b)
+    cand = torch.randint(0, V, (bs, T), generator=g).to(device)
+    cand[:, 1:] = pad.float().argmax(-1).view(bs, T)[:, :-1]
+    prefix = torch.arange(bs, dtype=torch.int32, device=device)
+    for a, b in zip(accept_greedy(candidates=cand, next_token_logits=odd, prefix_lens=prefix),
+                    accept_greedy(candidates=cand, next_token_logits=pad, prefix_lens=prefix)):
+        assert torch.equal(a, b)
+    info = W.info_to(W.sampling_info([1.0, 0.0, 0.7, 1.0], [0, 0, 20, 0], [0.95, 1.0, 0.9, 1.0]), device)
+    out = torch.full((bs * T, (V + 63) // 64 * 64), -1.0, device=device)
+    ref = target_probs(pad, info, bs=bs, T=T, out=out[:, :V])
+    raw = torch.full((bs * T * stride + 16,), -1.0, device=device)
+    got = target_probs(odd, info, bs=bs, T=T, out=raw[offset:].as_strided((bs * T, V), (stride, 1)))
+    assert torch.equal(got, ref)
+    assert bool((out[:, V:] == -1).all()) and int((raw == -1).sum()) == raw.numel() - bs * T * V
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_verify_long_history(device, dtype):
     # a history of 6000 tokens over 20483 ids: more vectors hold a penalised value than a
     # wave's LDS slots, so every lane penalises its own elements in place
