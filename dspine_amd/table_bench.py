@@ -1,9 +1,9 @@
 """Timing of the draft-side sampling table at a serving shape on one GPU: bs 64 requests x T 16
 (n = 960 block rows), K 16 lanes, H 4096, R 512, C 1024, V 151936, random bf16 / float32 inputs
 of those shapes (no checkpoint).  Prints one JSON line: microseconds per call and the matrix-core
-rate against MI355X's dense peak -- serial_rs_table in float32 (157.3 TFLOP/s), or with
-``--factor`` the factorized table in float64 (78.6 TFLOP/s; vocabulary 32768 there, the one-time
-cache build timed and reported beside it).
+rate against MI355X's dense peak -- serial_rs_table in bf16 parts of float32 operands (2.5 PFLOP/s),
+or with ``--factor`` the factorized table in float64 (78.6 TFLOP/s; vocabulary 32768 there, the
+one-time cache build timed and reported beside it).
 
     python -m dspine_amd.table_bench [--calls N] [--factor]
 """
@@ -14,15 +14,16 @@ import math
 
 import torch
 
-PEAK_TFLOPS = 157.3
+PEAK_TFLOPS = 2500.0
 PEAK_F64_TFLOPS = 78.6
 
 
 def flops(n, K, H, R, C):
-    """2 x multiply-adds of the three products: senders x [pg; pv], msg x write_w, and the dot
-    products with the candidates' head rows."""
+    """2 x multiply-adds of the three products -- senders x [pg; pv], msg x write_w, and the dot
+    products with the candidates' head rows -- in the bf16 parts they run as (three a float32
+    operand; six part products where both are float32)."""
     Ns = n * K
-    return 2.0 * (Ns * C * 2 * R + Ns * R * H + n * K * K * H)
+    return 2.0 * (3 * Ns * C * 2 * R + 6 * Ns * R * H + 3 * n * K * K * H)
 
 
 def factor_flops(n, K, H, R):
