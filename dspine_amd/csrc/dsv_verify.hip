@@ -3480,11 +3480,11 @@ __global__ __launch_bounds__(GA_THREADS) void k_greedy_accept(const ChunkStat* c
 // slot is loaded at once, the candidates under the largest such minimum drop out, and the others are
 // ranked among themselves by counting (9.5 us at 1088 rows of 8 bf16 lists of 20, where loading list
 // after list and selecting by radix took 12.3; 12.6 against 20.4 at 384 rows of 13 float32 lists of 33).
-// Selected by radix all the same: bf16 lists over TM_BF16 (five digits decide them: the call 76 us
-// against 82 at 64), rows of more slots than the registers take, rows left with over TM_RANK candidates.
+// Selected by radix all the same: bf16 lists over TM_BF16 (five digits decide them: the call 76.5 us
+// against 82 at 64, 73.9 against 75.0 at 40; by counting 72.9 against 73.5 at 33), rows of more slots than the registers take, rows left with over TM_RANK candidates.
 constexpr int TM_PER = 8;     // slots a thread holds
 constexpr int TM_RANK = 512;  // candidates ranked by counting
-constexpr int TM_BF16 = 40;
+constexpr int TM_BF16 = 33;
 template <int DT>
 __global__ __launch_bounds__(256) void k_topk_merge(const ChunkStat* cstat, const uint64_t* cand, int C, int kcand,
                                                     int32_t K, float* values_out, int64_t* ids_out, int sort_by_id) {
