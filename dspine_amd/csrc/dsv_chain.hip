@@ -788,18 +788,30 @@ __global__ __launch_bounds__(CH_THREADS) void k_chain(dsv_chain_args a) {
 
 // ---------------------------------------------------------------------------------------
 // Draft-side K-lane chain (kernels/dspine.py:616-674): a request's T-1 block rows, lanes the K
-// candidates, one workgroup per request.  A row's draw depends on the chain only through its sender,
-// the lane drawn on the row before.  Up to 16 lanes the workgroup evaluates every (row, sender) pair at
-// once (G lanes each, G the power of two from K up), walks the drawn lanes through LDS, and evaluates
-// the walked pairs again for the outputs.  Wider tables have too many pairs for that: their rows are
-// brought to LDS in batches and one wave walks them.  Bound by latency: a wave walking the rows from
-// memory took 46 us at 64 requests of 15 rows of 16 lanes (3 us a row) and 70 us at 16 rows of 32, this
-// 14 and 54; evaluating every pair at 32 lanes was slower than the wave's walk (the round's four calls
-// 104 us against 89).
+// candidates.  A row's draw depends on the chain only through its sender, the lane drawn on the row
+// before.  k_chain_walk takes the rows one after another, a wave a request: a memory latency and a
+// draw a row, 2 us at 16 lanes, 5.5 at 64, and the rest of the card is free for other requests.
+// k_chain_pairs (up to 16 lanes) gives a request a whole workgroup that evaluates every (row, sender)
+// pair at once (G lanes each, G the power of two from K up), walks the drawn lanes through LDS, and
+// evaluates the walked pairs again for the outputs: 14.8 us against 31.0 at 64 requests of 15 rows of 16
+// lanes, but it does K times the draws (55 against 33 at 1024 requests).  Rows brought to LDS for the
+// walk of wider tables were no faster than rows from memory at any size (17 to 32 lanes, 1 to 4096
+// requests) and 1.9 to 12 times slower from 384 requests on.
 // ---------------------------------------------------------------------------------------
 constexpr int SC_THREADS = 1024;
 constexpr int SC_PAIRS = 8192;  // (row, sender) pairs a batch holds
-constexpr int SC_TILE = 16384;  // table values a batch of the walk holds (a row of 64 lanes: 4096)
+
+// Whether the requests' workgroups of k_chain_pairs beat their waves: they cost about 5 us (8 lanes) or
+// 14 (16 lanes, 15 rows) for every 256 requests (a workgroup a CU), a wave 1.3 or 2 us a row whatever their
+// number.  Measured, pairs against walk in us at bs x rows: K 8: 256 x 2 5.6, 4.9 and x 3 5.7, 6.1;
+// 512 x 5 9.6, 8.8 and x 7 9.8, 11.3; 768 x 7 13.6, 11.5 and x 11 14.8, 16.8; 1024 x 11 19.2, 17.0 and
+// x 15 21.4, 21.9; 2048 x 31 57.5, 43.6.  K 16: 256 x 2 7.4, 6.2 and x 3 7.7, 8.2; 512 x 7 18.8, 16.4 and x 11
+// 24.1, 24.4; 768 x 63 137, 132.
+static bool sc_pairs(int64_t bs, int32_t K, int32_t rows) {
+  const int64_t rounds = (bs + 255) / 256;
+  if (K <= 8) return rounds <= 4 && rows >= 3 * rounds;
+  return K <= 16 && rounds <= 2 && rows >= (rounds == 1 ? 3 : 9);
+}
 
 struct ScDraw {
   float q, pmax;
@@ -831,12 +843,14 @@ __device__ __forceinline__ ScDraw sc_draw(float score, int l, int K, int32_t tk,
   // rank and mass ahead (ties: lower lane first)
   int rank = 0;
   float before = 0.f;
+  for (int d0 = 0; d0 < K; d0 += 8) {
 #pragma unroll
-  for (int d = 0; d < G; ++d) {  // (a lane past K holds -1: ahead of none)
-    const float pd = __shfl(p, d, G);
-    const bool ahead = pd > p || (pd == p && d < l);
-    rank += ahead;
-    before += ahead ? pd : 0.f;
+    for (int d = d0; d < d0 + 8; ++d) {  // (a lane past K holds -1: ahead of none)
+      const float pd = __shfl(p, d, G);
+      const bool ahead = pd > p || (pd == p && d < l);
+      rank += ahead;
+      before += ahead ? pd : 0.f;
+    }
   }
   const bool keep = live && rank < tk && before <= tp && p >= mp * pmax;
   const float w = keep ? p : 0.f;
@@ -859,56 +873,63 @@ __device__ __forceinline__ ScDraw sc_draw(float score, int l, int K, int32_t tk,
   return {q, pmax, choice < last ? choice : last};
 }
 
+// The rows of a greedy request: greedy_tok with a one-hot q; the chain is not read.
+__device__ __forceinline__ void sc_greedy(int64_t n0, int32_t K, int32_t tm1, const int64_t* cand,
+                                          const int64_t* greedy_tok, int64_t* out_tok, float* out_q) {
+  for (int64_t e = threadIdx.x; e < (int64_t)tm1 * K; e += blockDim.x) {
+    const int64_t n = n0 + e / K;
+    out_q[n * K + e % K] = cand[n * K + e % K] == greedy_tok[n] ? 1.f : 0.f;
+    if (e % K == 0) out_tok[n] = greedy_tok[n];
+  }
+}
+
+// One wave a request, its rows from memory one after another (the groups of a wave hold the same).
 template <int G>
-__global__ __launch_bounds__(SC_THREADS) void k_sample_chain(const float* table, int32_t K, int32_t tm1,
-                                                            const float* inv_temp, const int32_t* top_k,
-                                                            const float* top_p, const float* min_p,
-                                                            const int32_t* greedy, const float* u,
-                                                            const int64_t* cand, const int64_t* greedy_tok,
-                                                            int64_t* out_tok, float* out_q, float* confidence) {
+__global__ __launch_bounds__(WAVE) void k_chain_walk(const float* table, int32_t K, int32_t tm1, const float* inv_temp,
+                                                    const int32_t* top_k, const float* top_p, const float* min_p,
+                                                    const int32_t* greedy, const float* u, const int64_t* cand,
+                                                    const int64_t* greedy_tok, int64_t* out_tok, float* out_q,
+                                                    float* confidence) {
+  const int64_t b = blockIdx.x, n0 = b * tm1;
+  const int lane = threadIdx.x, l = lane % G, lc = l < K ? l : K - 1;
+  if (greedy[b] != 0) {
+    sc_greedy(n0, K, tm1, cand, greedy_tok, out_tok, out_q);
+    return;
+  }
+  const float inv_t = inv_temp[b], tp = top_p[b], mp = min_p[b];
+  const int32_t tk = top_k[b];
+  int sender = 0;
+  for (int64_t n = n0; n < n0 + tm1; ++n) {
+    const float x = __fmul_rn(table[(n * K + sender) * K + lc], inv_t);
+    const int64_t cl = cand[n * K + lc];
+    const ScDraw d = sc_draw<G>(l < K ? x : -INFINITY, l, K, tk, tp, mp, u[n]);
+    const int64_t tok = __shfl(cl, d.choice, G);
+    if (lane < K) out_q[n * K + l] = d.q;
+    if (lane == 0) {
+      out_tok[n] = tok;
+      if (confidence) confidence[n] = d.pmax;
+    }
+    sender = d.choice;
+  }
+}
+
+template <int G>
+__global__ __launch_bounds__(SC_THREADS) void k_chain_pairs(const float* table, int32_t K, int32_t tm1,
+                                                           const float* inv_temp, const int32_t* top_k,
+                                                           const float* top_p, const float* min_p,
+                                                           const int32_t* greedy, const float* u,
+                                                           const int64_t* cand, const int64_t* greedy_tok,
+                                                           int64_t* out_tok, float* out_q, float* confidence) {
   constexpr int NG = SC_THREADS / G;
   const int64_t b = blockIdx.x, n0 = b * tm1;
   const int tid = threadIdx.x, grp = tid / G, l = tid % G;
-  if (greedy[b] != 0) {  // greedy_tok with a one-hot q; the chain is not read
-    for (int64_t e = tid; e < (int64_t)tm1 * K; e += SC_THREADS) {
-      const int64_t n = n0 + e / K;
-      out_q[n * K + e % K] = cand[n * K + e % K] == greedy_tok[n] ? 1.f : 0.f;
-      if (e % K == 0) out_tok[n] = greedy_tok[n];
-    }
+  if (greedy[b] != 0) {
+    sc_greedy(n0, K, tm1, cand, greedy_tok, out_tok, out_q);
     return;
   }
   const float inv_t = inv_temp[b], tp = top_p[b], mp = min_p[b];
   const int32_t tk = top_k[b];
   const int lc = l < K ? l : K - 1;
-  if constexpr (G > 16) {
-    __shared__ float tile[SC_TILE], us[SC_TILE / 256];
-    __shared__ uint8_t drawn[SC_TILE / 256];  // (K > 16: at most SC_TILE / 289 rows a batch)
-    const int batch = SC_TILE / (K * K);
-    int sender = 0;
-    for (int i0 = 0; i0 < tm1; i0 += batch) {
-      const int rows = tm1 - i0 < batch ? tm1 - i0 : batch;
-      for (int e = tid; e < rows * K * K; e += SC_THREADS) tile[e] = table[(n0 + i0) * K * K + e];
-      if (tid < rows) us[tid] = u[n0 + i0 + tid];
-      __syncthreads();
-      if (tid < WAVE) {
-        for (int i = 0; i < rows; ++i) {
-          const int64_t n = n0 + i0 + i;
-          const float x = __fmul_rn(tile[(i * K + sender) * K + lc], inv_t);
-          const ScDraw d = sc_draw<G>(l < K ? x : -INFINITY, l, K, tk, tp, mp, us[i]);
-          if (tid < K) out_q[n * K + l] = d.q;
-          if (tid == 0) {
-            drawn[i] = (uint8_t)d.choice;
-            if (confidence) confidence[n] = d.pmax;
-          }
-          sender = d.choice;
-        }
-      }
-      __syncthreads();
-      if (tid < rows) out_tok[n0 + i0 + tid] = cand[(n0 + i0 + tid) * K + drawn[tid]];
-      __syncthreads();
-    }
-    return;
-  }
   __shared__ uint8_t drawn[SC_PAIRS], senders[SC_PAIRS];
   __shared__ int s_sender;
   auto score = [&](int64_t n, int sender) {
@@ -951,7 +972,6 @@ __global__ __launch_bounds__(SC_THREADS) void k_sample_chain(const float* table,
     __syncthreads();
   }
 }
-
 
 // ---------------------------------------------------------------------------------------
 // Sparse joint target (sampling/sparse/target.py:22-66, CPU form :156-178).  One wave per row
@@ -1239,14 +1259,15 @@ extern "C" int dsv_sample_chain(const float* table, int64_t n, int32_t K, int32_
   const int64_t bs = n / (block_size - 1);
   if (bs == 0) return DSV_OK;
   if (bs > 2147483647ll) DSV_FAIL(DSV_ERR_INVALID, "dsv_sample_chain: too many chains");
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3((unsigned)bs), dim3(SC_THREADS), 0, stream, table, K, block_size - 1, inv_temp,
+  auto launch = [&](auto kernel, int threads) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)bs), dim3(threads), 0, stream, table, K, block_size - 1, inv_temp,
                        top_k, top_p, min_p, greedy, u, cand, greedy_tok, out_tok, out_q, confidence);
   };
-  if (K <= 8) launch(k_sample_chain<8>);
-  else if (K <= 16) launch(k_sample_chain<16>);
-  else if (K <= 32) launch(k_sample_chain<32>);
-  else launch(k_sample_chain<64>);
+  const bool pairs = sc_pairs(bs, K, block_size - 1);
+  if (K <= 8) pairs ? launch(k_chain_pairs<8>, SC_THREADS) : launch(k_chain_walk<8>, WAVE);
+  else if (K <= 16) pairs ? launch(k_chain_pairs<16>, SC_THREADS) : launch(k_chain_walk<16>, WAVE);
+  else if (K <= 32) launch(k_chain_walk<32>, WAVE);
+  else launch(k_chain_walk<64>, WAVE);
   DSV_CHECK_LAUNCH("dsv_sample_chain");
   return DSV_OK;
 }

@@ -85,7 +85,8 @@ def serial_sample_chain(table, inv_temp, top_k, top_p, min_p, greedy, u, cand, g
     q = w / sum w; the drawn lane is #(cdf <= u * total) clamped to the last kept lane.  Greedy
     requests emit greedy_tok with a one-hot q.  ``confidence_out`` float32 [>=n] receives max p
     (before filtering) of each row of a non-greedy request; other entries are left as they are.
-    One wavefront per request walks its chain; K <= 64."""
+    A wave walks a request's rows, or (K <= 16, batches the card holds in a few rounds) a workgroup draws
+    every (row, sender) pair at once; K <= 64."""
     t = int(block_size)
     n, k = cand.shape
     if t < 2 or n % (t - 1) or tuple(table.shape) != (n, k, k) or not table.is_contiguous():

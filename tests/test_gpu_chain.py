@@ -703,7 +703,7 @@ def test_sample_chain_matches_oracle(device, seed):
 @pytest.mark.parametrize("k,T", [(1, 4), (8, 3), (9, 17), (16, 2), (16, 515), (17, 60), (32, 18), (33, 16), (64, 7)])
 def test_sample_chain_widths(device, k, T):
     """Every group width (8, 16, 32, 64 lanes) at its edges, chains that fill more than one batch of
-    rows (512 rows of 16 lanes; 56 of 17, 16 of 32, 15 of 33, 4 of 64), a greedy request among them."""
+    rows (512 rows of 16 lanes), a greedy request among them."""
     O = _O()
     params = [(1.0, k, 1.0, 0.0, 0), (0.7, max(1, k // 2), 0.8, 0.05, 0), (1.0, k, 1.0, 0.0, 1)]
     table, cand, greedy_tok, u = _chain_inputs(len(params), T, k, 7 * k + T)
@@ -715,6 +715,30 @@ def test_sample_chain_widths(device, k, T):
     assert np.array_equal(out_tok.numpy(), ref_tok)
     torch.testing.assert_close(out_q, torch.as_tensor(ref_q), rtol=1e-5, atol=1e-6)
     torch.testing.assert_close(conf.cpu(), torch.as_tensor(conf_ref), rtol=1e-5, atol=1e-6)
+
+
+@pytest.mark.parametrize("k,T,few,many", [(4, 4, 256, 257), (8, 13, 1024, 1025), (9, 4, 256, 257), (16, 10, 512, 513),
+                                          (16, 3, 2, 300)])
+def test_sample_chain_batch_sizes(device, k, T, few, many):
+    """Requests drawn pair by pair by a workgroup each, and walked by a wave each in a batch one request
+    larger (two-row chains: walked in both): the same bits, and the oracle's on the last requests."""
+    O = _O()
+    kinds = [(1.0, k, 1.0, 0.0, 0), (0.7, max(1, k // 2), 0.8, 0.05, 0), (1.0, k, 1.0, 0.0, 1), (1.3, k, 0.9, 0.0, 0)]
+    g = torch.Generator().manual_seed(k * T)
+    n, r = many * (T - 1), few * (T - 1)
+    table = torch.randn(n, k, k, generator=g) * 3.0
+    cand = torch.randint(0, 1 << 40, (n, k), generator=g).sort(-1).values
+    gtok, u = cand[:, k // 2].clone(), torch.rand(n, generator=g)
+    staged = _staged([kinds[b % 4] for b in range(many)])
+    conf = [torch.full((m,), -0.5, device=device) for m in (n, r)]
+    tok, q = _run_chain(device, table, staged, u, cand, gtok, T, confidence=conf[0])
+    tok2, q2 = _run_chain(device, table[:r], [x[:few] for x in staged], u[:r], cand[:r], gtok[:r], T, confidence=conf[1])
+    assert torch.equal(tok[:r], tok2) and torch.equal(q[:r], q2) and torch.equal(conf[0][:r], conf[1])
+    at = slice((many - 8) * (T - 1) if many > 8 else 0, n)
+    last = [x[-8:] for x in staged]
+    ref_tok, ref_q = O.sample_chain(*_np(table[at], *last, u[at], cand[at], gtok[at]), T)
+    assert np.array_equal(tok[at].numpy(), ref_tok)
+    torch.testing.assert_close(q[at], torch.as_tensor(ref_q), rtol=1e-5, atol=1e-6)
 
 
 def test_sample_chain_ties_break_to_lower_lane(device):
