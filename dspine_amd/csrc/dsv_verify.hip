@@ -3418,60 +3418,90 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
 // ---------------------------------------------------------------------------------------
 // Greedy verify (verification/caps.py:32-59, verification/ragged.py:51-76)
 // ---------------------------------------------------------------------------------------
-// First argmax of a row from its chunks' maxima, by a wave: the first chunk holding the largest (0 if
-// none exceeds -inf).
-__device__ __forceinline__ int32_t chunk_argmax(const ChunkStat* cs, int C, int lane) {
+// First argmax of a row from its chunks' maxima, by a group of G lanes (1, 2, 4, 8, 16 or the wave; lane
+// l of it): the first chunk holding the largest (0 if none exceeds -inf).
+__device__ __forceinline__ int32_t chunk_argmax(const ChunkStat* cs, int C, int G, int l) {
   float M = -INFINITY;
   int32_t arg = 0;
-  for (int c0 = 0; c0 < C; c0 += WAVE) {
-    const bool in = c0 + lane < C;
-    const ChunkStat* s = cs + (in ? c0 + lane : 0);
+  for (int c0 = 0; c0 < C; c0 += G) {  // (one round but where the group is the wave)
+    const bool in = c0 + l < C;
+    const ChunkStat* s = cs + (in ? c0 + l : 0);
     const float m = in ? s->m : -INFINITY;
     const int32_t at = s->arg;
-    const float mx = wave_max_f32(m);
-    if (!(mx > M)) continue;
-    M = mx;
-    arg = readlane_at(at, __ffsll((unsigned long long)__ballot(m == mx)) - 1);
+    float mx = m;
+    if (G == WAVE) {
+      mx = wave_max_f32(m);
+    } else {
+      if (G > 1) mx = fmaxf(mx, dpp<DPP_QUAD_XOR1>(mx, mx));
+      if (G > 2) mx = fmaxf(mx, dpp<DPP_QUAD_XOR2>(mx, mx));
+      if (G > 4) mx = fmaxf(mx, dpp<DPP_ROW_HALF_MIRROR>(mx, mx));
+      if (G > 8) mx = fmaxf(mx, dpp<DPP_ROW_MIRROR>(mx, mx));
+    }
+    const uint64_t hit = __ballot(m == mx);
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int32_t best = __shfl(at, __ffsll((unsigned long long)(hit & (~0ull << (lane - l)))) - 1, WAVE);
+    if (mx > M) M = mx, arg = best;
   }
   return arg;
 }
 
-// Greedy acceptance, one workgroup per request, a wave per row: every row's argmax at once.  (One lane
-// walking the request's rows and chunks one load after another took 23.6 us at 1 x 17 rows of 13
-// chunks, this 3.0.)
+// Greedy acceptance, one workgroup per request with the waves its rows need, G lanes a row: every row's
+// argmax at once, rows that fit one wave without LDS.  (One lane walking the request's rows and chunks
+// one load after another took 23.6 us at 1 x 17 rows of 13 chunks, this 3.0.  Bound by latency, and by the
+// workgroups' launch in large batches: with 16 waves whatever the rows, the call took 29.0 us at 4096
+// requests of one row of one chunk, so 19.5, with the walking lane 18.5.)
 constexpr int GA_THREADS = 1024;
 constexpr int GA_ROWS = 1024;  // argmaxes kept in LDS
-__global__ __launch_bounds__(GA_THREADS) void k_greedy_accept(const ChunkStat* cstat, int C, const int64_t* cand,
-                                                             const int32_t* lens, int32_t cap_static,
-                                                             const int32_t* prefix, int32_t T, int32_t* accept,
-                                                             int32_t* commit, int64_t* bonus, int64_t* output,
-                                                             int32_t* new_seq, int64_t* top1_out) {
+__global__ __launch_bounds__(GA_THREADS) void k_greedy_accept(const ChunkStat* cstat, int C, int G,
+                                                             const int64_t* cand, const int32_t* lens,
+                                                             int32_t cap_static, const int32_t* prefix, int32_t T,
+                                                             int32_t* accept, int32_t* commit, int64_t* bonus,
+                                                             int64_t* output, int32_t* new_seq, int64_t* top1_out) {
   __shared__ int32_t top1[GA_ROWS];
   __shared__ int s_acc;
   const int64_t b = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid / WAVE;
+  const int tid = threadIdx.x, threads = blockDim.x, grp = tid / G, l = tid & (G - 1);
+  const int32_t before = prefix[b];
   int cap = lens ? lens[b] : cap_static;
   cap = cap < 1 ? 1 : (cap > T ? T : cap);
-  if (tid == 0) s_acc = cap - 1;
-  __syncthreads();
-  const int rows = top1_out ? T : cap;
-  for (int i = w; i < rows; i += GA_THREADS / WAVE) {
-    const int32_t arg = chunk_argmax(cstat + (b * T + i) * C, C, lane);
-    if (lane) continue;
-    if (i < GA_ROWS) top1[i] = arg;
-    if (top1_out) top1_out[b * T + i] = arg;
-    if (i < cap - 1 && cand[b * T + i + 1] != arg) atomicMin(&s_acc, i);
+  int acc;
+  int64_t bon;
+  if (T * (int64_t)G <= WAVE) {  // a lane group for every row
+    const int i = grp < T ? grp : T - 1;
+    const int64_t next = i < T - 1 ? cand[b * T + i + 1] : 0;
+    const int32_t arg = chunk_argmax(cstat + (b * T + i) * C, C, G, l);
+    const uint64_t miss = __ballot(i < cap - 1 && next != arg);
+    acc = miss ? (__ffsll((unsigned long long)miss) - 1) / G : cap - 1;
+    bon = __shfl(arg, acc * G, WAVE);
+    if (l == 0 && grp < T) {
+      output[b * T + i] = i == acc ? bon : next;
+      if (top1_out) top1_out[b * T + i] = arg;
+    }
+  } else {
+    if (tid == 0) s_acc = cap - 1;
+    __syncthreads();
+    const int rows = top1_out ? T : cap;
+    for (int i0 = 0; i0 < rows; i0 += threads / G) {
+      const int i = i0 + grp < rows ? i0 + grp : rows - 1;  // (a group past the last row repeats it)
+      const int64_t next = i < cap - 1 ? cand[b * T + i + 1] : 0;
+      const int32_t arg = chunk_argmax(cstat + (b * T + i) * C, C, G, l);
+      if (l == 0) {
+        if (i < GA_ROWS) top1[i] = arg;
+        if (top1_out) top1_out[b * T + i] = arg;
+        if (i < cap - 1 && next != arg) atomicMin(&s_acc, i);
+      }
+    }
+    __syncthreads();
+    acc = s_acc;
+    bon = acc < GA_ROWS ? top1[acc] : chunk_argmax(cstat + (b * T + acc) * C, C, G, l);
+    for (int i = tid; i < T; i += threads)
+      output[b * T + i] = i == acc ? bon : (i < T - 1 ? cand[b * T + i + 1] : 0);
   }
-  __syncthreads();
-  const int acc = s_acc;
-  const int64_t bon = acc < GA_ROWS ? top1[acc] : chunk_argmax(cstat + (b * T + acc) * C, C, lane);
-  for (int i = tid; i < T; i += GA_THREADS)
-    output[b * T + i] = i == acc ? bon : (i < T - 1 ? cand[b * T + i + 1] : 0);
   if (tid == 0) {
     accept[b] = acc;
     commit[b] = acc + 1;
     bonus[b] = bon;
-    new_seq[b] = prefix[b] + acc + 1;
+    new_seq[b] = before + acc + 1;
   }
 }
 
@@ -3969,8 +3999,12 @@ static int greedy_launch(const void* logits, int32_t dtype, int64_t rows, int64_
   if (prof && hipEventRecord(g_prof_stop, stream) != hipSuccess)
     DSV_FAIL(DSV_ERR_LAUNCH, "dsv_greedy_verify: cannot record the profiling stop event");
   DSV_CHECK_LAUNCH("k_chunk");
-  hipLaunchKernelGGL(k_greedy_accept, dim3((unsigned)bs), dim3(GA_THREADS), 0, stream, P.cstat, P.C, candidates,
-                     verify_lens, cap, prefix_lens, T, accept, commit, bonus, output, new_seq, top1_out);
+  int G = 1;  // lanes a row
+  while (G < P.C && G < WAVE) G = G < 16 ? 2 * G : WAVE;
+  const int64_t waves = ((int64_t)T * G + WAVE - 1) / WAVE;
+  hipLaunchKernelGGL(k_greedy_accept, dim3((unsigned)bs), dim3(waves * WAVE < GA_THREADS ? (int)waves * WAVE : GA_THREADS),
+                     0, stream, P.cstat, P.C, G, candidates, verify_lens, cap, prefix_lens, T, accept, commit, bonus,
+                     output, new_seq, top1_out);
   DSV_CHECK_LAUNCH("k_greedy_accept");
   return DSV_OK;
 }

@@ -211,6 +211,38 @@ def test_greedy_edges(device, bs, T, V, dtype):
         assert top is None or np.array_equal(top.cpu().numpy().reshape(-1), np.asarray(top1).reshape(-1))
 
 
+@pytest.mark.parametrize("T,V", [(64, 64), (65, 64), (32, 20481), (33, 20481), (16, 61441), (8, 102401), (9, 102401),
+                                 (4, 163841), (5, 163841), (1, 327681), (2, 327681)])
+def test_greedy_lane_groups(device, T, V):
+    """Every width of the accept kernel's lane groups (1, 2, 4, 8, 16 lanes and the wave a row) with the
+    rows that just fit one wave and those that just do not: maxima tied over all chunks, or one in a
+    chunk of its own, caps and verify lengths, with the argmaxes and without."""
+    from dspine_amd.verification.caps import accept_greedy
+
+    O = _oracle()
+    g = torch.Generator().manual_seed(T)
+    bs = 5
+    logits = torch.randint(-60, 60, (bs * T, V), generator=g).to(torch.bfloat16)
+    logits[torch.arange(1, bs * T, 2), torch.randint(0, V, (bs * T // 2,), generator=g)] = 64.0
+    top1 = O.argmax_rows(logits)
+    cand = torch.zeros(bs, T, dtype=torch.int64)
+    cand[:, 1:] = torch.as_tensor(top1).view(bs, T)[:, : T - 1]
+    for b in range(1, bs):  # the first request's drafts are all accepted
+        if T > 1:
+            cand[b, int(torch.randint(1, T, (1,), generator=g))] += 1
+    prefix = torch.arange(bs, dtype=torch.int32)
+    lens = torch.randint(1, T + 1, (bs,), generator=g).to(torch.int32)
+    x, c, p = logits.to(device), cand.to(device), prefix.to(device)
+    for vl in (None, lens):
+        ref = O.greedy_accept(top1, cand.numpy(), [T] * bs if vl is None else vl.tolist(), prefix.numpy())
+        for top in (None, torch.full((bs, T), -1, dtype=torch.int64, device=device)):
+            outs = accept_greedy(candidates=c, next_token_logits=x, prefix_lens=p, top1=top,
+                                 **({"cap": T} if vl is None else {"verify_lens": vl.to(device)}))
+            for got, r in zip(outs, ref):
+                assert np.array_equal(got.cpu().numpy(), r)
+            assert top is None or np.array_equal(top.cpu().numpy().reshape(-1), np.asarray(top1).reshape(-1))
+
+
 # ------------------------------------------------------------------------------------------
 # fused sampled verify
 # ------------------------------------------------------------------------------------------
