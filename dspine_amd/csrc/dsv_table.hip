@@ -86,16 +86,22 @@ __device__ __forceinline__ f4 mfma(u4 a, u4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bh8, a), __builtin_bit_cast(bh8, b), c, 0, 0, 0);
 }
 
-// x = hi + mid + lo, each bf16 (8 significant bits, round to nearest even): exact for every finite
-// float32 above the underflow of its last bits.  An infinite x is (inf, finite, 0): its products
-// stay infinite.  Two values a call, packed.
+// x = hi + mid + lo, each bf16 (8 significant bits, round to nearest even): exact for finite float32 of
+// 2^-110 and above (below, lo and then mid end under the smallest bf16: 16 bits are left at 2^-118, 8 at
+// 2^-126).  hi is held to the largest bf16, so that a finite x above it stays finite against a zero; an
+// infinite x is (largest, inf, finite): its product with a bf16 operand is the infinity or, against zero,
+// the NaN that it is.  (Against a second split operand it may be NaN for inf, in ref alone: an infinite
+// ref makes its dot products over its norm NaN either way.)  Two values a call, packed.
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
-  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{a, b}), bh2));
-  const float ra = fmaxf(a - __uint_as_float(hi << 16), -1e36f);  // (inf - inf is NaN: the bound)
-  const float rb = fmaxf(b - __uint_as_float(hi & 0xFFFF0000u), -1e36f);
+  const float top = __uint_as_float(0x7F7F0000u);  // the largest bf16
+  hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{__builtin_amdgcn_fmed3f(a, -top, top),
+                                                                __builtin_amdgcn_fmed3f(b, -top, top)}), bh2));
+  const float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xFFFF0000u);
   mid = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{ra, rb}), bh2));
-  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(
-                                        (f2{ra - __uint_as_float(mid << 16), rb - __uint_as_float(mid & 0xFFFF0000u)}), bh2));
+  // (inf - inf is NaN: the bound, below every finite x's lo)
+  const float la = fmaxf(ra - __uint_as_float(mid << 16), -1e34f);
+  const float lb = fmaxf(rb - __uint_as_float(mid & 0xFFFF0000u), -1e34f);
+  lo = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{la, lb}), bh2));
 }
 __device__ __forceinline__ void split8(const f4& x, const f4& y, u4& hi, u4& mid, u4& lo) {
   uint32_t h, m, l;

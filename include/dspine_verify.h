@@ -377,7 +377,8 @@ int dsv_sps_plan(const float* raw, int64_t raw_stride, int32_t bs, int32_t gamma
                  int32_t* qo_indptr, int64_t* window_index, dsv_stream_t stream);
 
 /* Draft-side sampling table of the serial last-write refinement (kernels/dspine.py:505-613,  */
-/* serial_rs_table), float32 accuracy on the matrix cores (three bf16 parts a float32 operand): */
+/* serial_rs_table), float32 accuracy on the matrix cores (three bf16 parts a float32 operand, */
+/* exact from 2^-110 up to the largest float; weights and messages below lose last bits):      */
 /* out [n, K, K] with n = bs * (T - 1) block                                                   */
 /* rows, out[n, j, c] = normalize(raw[r] + rms[r] * ((sigmoid(query[r] + e_j pg^T + gb) *     */
 /* (e_j pv^T + res_j res_proj^T)) write_w^T)) * norm_w . head[n, c], r = the row's state row,  */

@@ -114,6 +114,34 @@ def test_table_infinite_weight_saturates_the_gate(device):
     torch.testing.assert_close(table.double(), _ref(d, T), rtol=1e-4, atol=1e-4)
 
 
+@pytest.mark.parametrize("big", [torch.finfo(torch.float32).max, 3.397e38, 3.389e38])
+def test_table_weights_at_the_end_of_float32(device, big):
+    """Finite weights above the largest bf16 (3.3895e38) stay finite: against codes and residual codes of
+    zero they add nothing, against the smallest ones what they are worth, in every weight matrix."""
+    T = 3
+    d = _inputs(11, bs=2, T=T, H=64, R=64, C=32, V=64, k=4, residual=True)
+    zero, tiny = slice(0, 3), slice(3, 5)
+    d["codebook"][:, zero], d["res_emb"][:, zero] = 0.0, 0.0
+    d["codebook"][:, tiny] = torch.sign(d["codebook"][:, tiny].float()).to(torch.bfloat16) * 2.0 ** -126
+    for name in ("pg", "pv", "res_proj"):
+        d[name][::7, zero] = big
+        d[name][1::7, zero] = -big
+    for name in ("pg", "pv"):
+        d[name][2::7, tiny] = big / 2 ** 3
+        d[name][3::7, 3] = -big
+    d["pv"][9] = 0.0  # a column of the message that is zero, and one near 2^-10
+    d["res_proj"][9] = 0.0
+    d["w_last"][:, 9] = big
+    d["pv"][10] *= 2.0 ** -10
+    d["res_proj"][10] *= 2.0 ** -10
+    d["res_proj"][10, zero] = 0.0
+    d["w_last"][5, 10] = big
+    d["rms"] *= 2.0 ** -116  # (every other write is lost in the state: that one is of its size)
+    table = _gpu_table(d, T, device).cpu()
+    assert torch.isfinite(table).all()
+    torch.testing.assert_close(table.double(), _ref(d, T), rtol=1e-4, atol=1e-4)
+
+
 def test_table_residual_and_candidate_head(device):
     """The terminal residual added to the value, and head rows given per candidate
     ([n, K, H] instead of lm_head gathered by id)."""
