@@ -90,8 +90,9 @@ def test_table_candidate_widths(device, k):
     (2, 9, 256, 192, 64, 48, 1.0),    # three lane blocks
 ])
 def test_table_tile_edges(device, bs, T, H, R, C, k, scale):
-    """Sizes that end inside the kernels' tiles (128 senders, 256 h, 64 k), in the 2-norm: float32
-    sums of C, R and H terms round to about 2^-24 (sqrt(C) + sqrt(R) + sqrt(H)) of their size."""
+    """Small batches (16 message columns a workgroup, 64-h tiles) of sizes that end inside the kernels'
+    tiles (128 senders, 64 h, 64 k), in the 2-norm: float32 sums of C, R and H terms round to about
+    2^-24 (sqrt(C) + sqrt(R) + sqrt(H)) of their size."""
     d = _inputs(31, bs=bs, T=T, H=H, R=R, C=C, V=512, k=k)
     d["w_last"] = d["w_last"] * scale
     d["rms"] = d["rms"] / scale
@@ -100,6 +101,35 @@ def test_table_tile_edges(device, bs, T, H, R, C, k, scale):
     bound = 2.0 ** -24 * (math.sqrt(C) + math.sqrt(R) + math.sqrt(H))
     assert float((table - ref).norm() / ref.norm()) < bound
     assert torch.isfinite(table).all()
+
+
+@pytest.mark.parametrize("bs,T,H,R,C,k,residual,cand_head", [
+    (27, 6, 4112, 128, 80, 16, False, False),   # 256-h tiles, one lane block: nine slices, the last of 16 h
+    (14, 6, 4112, 64, 32, 17, True, False),     # two lane blocks, 140 units (17 and a half workgroups)
+    (9, 6, 4240, 64, 32, 40, False, True),      # three lane blocks, a slice that ends inside its second tile
+    (7, 6, 4112, 64, 144, 64, False, False),    # four lane blocks
+    (409, 6, 272, 64, 16, 5, True, True),       # one slice of two tiles
+    (60, 6, 272, 512, 80, 16, True, False),     # 64 message columns: 37 and a half sender blocks x 8
+    (86, 6, 1040, 512, 272, 12, False, True),   # both
+])
+def test_table_large_batches(device, bs, T, H, R, C, k, residual, cand_head):
+    """The kernels of batches that fill the card: 256-h tiles where (units / 8) x (H / 256) is 256 or more,
+    64 message columns a workgroup where (senders / 128) x (R / 64) is, at sizes that end inside a tile,
+    a slice and a sender block.  The bound is the one above; for the largest of up to 10^6 elements, 5
+    deviations, three times that where one sender's norm is that much larger than the mean."""
+    d = _inputs(17, bs=bs, T=T, H=H, R=R, C=C, V=256, k=k, residual=residual)
+    n, units = d["cand"].shape[0], d["cand"].shape[0] * -(-k // 16)
+    wide, columns = -(-units // 8) * -(-H // 256), -(-n * k // 128) * (R // 64)
+    assert wide >= 256 or columns >= 256
+    head = None
+    if cand_head:
+        g = torch.Generator().manual_seed(9)
+        head = (torch.randn(n, k, H, generator=g) / math.sqrt(H)).to(torch.bfloat16)
+    table = _gpu_table(d, T, device, candidate_head=head).cpu().double()
+    ref = _ref(d, T, candidate_head=head)
+    bound = 2.0 ** -24 * (math.sqrt(C) + math.sqrt(R) + math.sqrt(H))
+    assert float((table - ref).norm() / ref.norm()) < bound
+    assert float((table - ref).abs().max() / ref.square().mean().sqrt()) < 16 * bound
 
 
 def test_table_infinite_weight_saturates_the_gate(device):
