@@ -502,17 +502,18 @@ __global__ void k_rs_finish(RsArgs A) {
 
 using namespace dsv;
 
-// The table's tile and H slices.  256-h tiles of eight waves (one workgroup a CU) where they fill the
-// card; below that 64-h tiles of two waves, two workgroups a CU, which spread a small batch over more
-// of it (15 rows, H 4096, R 512: k_rs_table 25 us against 37; 120 rows, the call 88 us against 118; 240
-// rows, the last batch under the line, 127 against 144).
+// The table's tile and H slices.  256-h tiles of eight waves (one workgroup a CU) from where they keep more
+// than half of the card busy; below that 64-h tiles of two waves, two workgroups a CU, which spread a small
+// batch over more of it.  The call at 16 lanes, narrow against wide in us, by wide tiles: H 4096, R 512 64
+// tiles (30 rows) 58, 70; 128: 68, 72; 192: 87, 79; 240: 90, 84; 480: 156, 132.  H 2048, R 256 120: 42, 46;
+// 136: 54, 48.  H 1024 120: 42, 46; 136: 55, 51.  32 lanes 128: 67, 75; 240: 96, 88.  64 lanes 240: 111, 112.
 struct RsPlan {
   int tile, slices, hs;
 };
 static RsPlan rs_plan(int64_t units, int32_t H) {
   const int64_t blocks = (units + RS_B / 16 - 1) / (RS_B / 16);
   RsPlan p;
-  p.tile = blocks * ((H + 255) / 256) >= 256 ? 256 : 64;
+  p.tile = blocks * ((H + 255) / 256) > 128 ? 256 : 64;
   const int64_t slots = p.tile == 256 ? 256 : 512, tiles = (H + p.tile - 1) / p.tile;
   const int64_t want = blocks >= slots ? 1 : slots / blocks;
   p.slices = (int)(want < tiles ? want : tiles);

@@ -88,6 +88,7 @@ def test_table_candidate_widths(device, k):
     (5, 6, 1040, 128, 144, 24, 1e18),  # weights far from 1: the parts keep float32's exponents
     (13, 2, 528, 512, 272, 9, 1e-18),
     (2, 9, 256, 192, 64, 48, 1.0),    # three lane blocks
+    (32, 3, 4096, 64, 16, 16, 1.0),   # the largest batch of 64-h tiles
 ])
 def test_table_tile_edges(device, bs, T, H, R, C, k, scale):
     """Small batches (16 message columns a workgroup, 64-h tiles) of sizes that end inside the kernels'
@@ -104,6 +105,7 @@ def test_table_tile_edges(device, bs, T, H, R, C, k, scale):
 
 
 @pytest.mark.parametrize("bs,T,H,R,C,k,residual,cand_head", [
+    (33, 3, 4096, 64, 16, 16, False, False),    # the smallest batch of 256-h tiles
     (27, 6, 4112, 128, 80, 16, False, False),   # 256-h tiles, one lane block: nine slices, the last of 16 h
     (14, 6, 4112, 64, 32, 17, True, False),     # two lane blocks, 140 units (17 and a half workgroups)
     (9, 6, 4240, 64, 32, 40, False, True),      # three lane blocks, a slice that ends inside its second tile
@@ -113,14 +115,14 @@ def test_table_tile_edges(device, bs, T, H, R, C, k, scale):
     (86, 6, 1040, 512, 272, 12, False, True),   # both
 ])
 def test_table_large_batches(device, bs, T, H, R, C, k, residual, cand_head):
-    """The kernels of batches that fill the card: 256-h tiles where (units / 8) x (H / 256) is 256 or more,
+    """The kernels of batches that fill the card: 256-h tiles where (units / 8) x (H / 256) is over 128,
     64 message columns a workgroup where (senders / 128) x (R / 64) is, at sizes that end inside a tile,
     a slice and a sender block.  The bound is the one above; for the largest of up to 10^6 elements, 5
     deviations, three times that where one sender's norm is that much larger than the mean."""
     d = _inputs(17, bs=bs, T=T, H=H, R=R, C=C, V=256, k=k, residual=residual)
     n, units = d["cand"].shape[0], d["cand"].shape[0] * -(-k // 16)
     wide, columns = -(-units // 8) * -(-H // 256), -(-n * k // 128) * (R // 64)
-    assert wide >= 256 or columns >= 256
+    assert wide > 128 or columns >= 256
     head = None
     if cand_head:
         g = torch.Generator().manual_seed(9)
