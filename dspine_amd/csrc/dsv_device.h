@@ -65,7 +65,6 @@ constexpr int BCT = 256;             // threads of the bonus / finalize kernels
 constexpr int QMAX = 64;             // largest supported sparse-q width K
 constexpr int FLAG_FULL_HIST = 2;    // nucleus row whose cut needs the full value histogram
 constexpr int FLAG_SCAN_DRAW = 4;    // dense row whose bonus draw k_final plans from a scan of every chunk
-constexpr int FLAG_TIES_COUNTED = 8; // full-histogram row whose chunks' counts of cut-key values are in rties
 constexpr int SJ_CAP = 32;           // packed capacity of the sparse joint target (sampling/target.py:84-87)
 
 // Row data of the probability filter: float32 probabilities taken as they are, where the other row
@@ -209,13 +208,13 @@ __device__ __forceinline__ uint4 load_vec(const char* rowp, int64_t vi, int64_t 
 }
 // The same for rows of any alignment: whole vectors in one load all the same.  (Loading them element by
 // element, the top 20 of 544 rows of 151931 bf16 logits took 111 us, so 51.)
+__device__ __forceinline__ uint4 load_any(const char* rowp, int64_t vi) {
+  const v4u_t t = __builtin_nontemporal_load(reinterpret_cast<const v4u2_t*>(rowp + vi * 16));
+  return make_uint4(t.x, t.y, t.z, t.w);
+}
 template <int DT>
 __device__ __forceinline__ uint4 load_vec_any(const char* rowp, int64_t vi, int64_t hi) {
-  if ((vi + 1) * Elems<DT>::n <= hi) {
-    const v4u_t t = __builtin_nontemporal_load(reinterpret_cast<const v4u2_t*>(rowp + vi * 16));
-    return make_uint4(t.x, t.y, t.z, t.w);
-  }
-  return load_vec<DT>(rowp, vi, hi, false);
+  return (vi + 1) * Elems<DT>::n <= hi ? load_any(rowp, vi) : load_vec<DT>(rowp, vi, hi, false);
 }
 
 // An empty asm that claims to rewrite the registers: values unpacked from them before the

@@ -1977,7 +1977,6 @@ __device__ __forceinline__ void nuc_row_f32(const KParams& P, int64_t r, F32NucL
       rs.S_kept = (double)(L.pmass[0][0] + L.mass[0][0]) / fx;
     }
     rs.S_f = (float)rs.S_kept;
-    if (count_ties) rs.flags |= FLAG_TIES_COUNTED;
     nucleus_finish<DT>(P, r, b, s, rs, T, xt, tok, tie_tok, ro);
   }
   __syncthreads();
@@ -3078,128 +3077,14 @@ __global__ __launch_bounds__(FCT) void k_final(KParams P) {
 }
 
 // ---------------------------------------------------------------------------------------
-// The target distribution of one (row, chunk) written out densely with each thread a span of
-// consecutive ids (runtime/worker.py:440-508): the ordered path of k_dense_p -- rows whose cut
-// keeps only some of the values at the cut key (their rank in id order decides), and outputs
-// that are not 4-byte aligned.
-// ---------------------------------------------------------------------------------------
-template <int DT, bool ALIGNED>
-__device__ __forceinline__ void dense_p_spans(const KParams& P, int64_t r, int c, int b, const RowSum& rs, int mode,
-                                              float* out, int64_t out_stride) {
-  constexpr int CV = Elems<DT>::cv, CHE = Elems<DT>::chunk, FE = CV * Elems<DT>::n;
-  constexpr int NW = CT / WAVE;
-  __shared__ int32_t red_i[NW];
-  __shared__ ListEntry lst[DSV_LIST_K];
-  __shared__ int32_t s_before;
-  const dsv_verify_args& a = P.a;
-  const int tid = threadIdx.x;
-  const int64_t V = a.vocab;
-  const int64_t jlo = (int64_t)c * CHE + (int64_t)tid * FE;
-  float* orow = out + r * out_stride;
-  // the span's values, four at a time
-  float4 acc4 = make_float4(0.f, 0.f, 0.f, 0.f);
-  auto put = [&](int i, float v) {
-    const int k = i & 3;
-    if (k == 0) acc4.x = v; else if (k == 1) acc4.y = v; else if (k == 2) acc4.z = v; else acc4.w = v;
-    if (k == 3) {
-      const int64_t j = jlo + i - 3;
-      if (j + 3 < V) {
-        *reinterpret_cast<float4*>(orow + j) = acc4;
-      } else {
-        if (j < V) orow[j] = acc4.x;
-        if (j + 1 < V) orow[j + 1] = acc4.y;
-        if (j + 2 < V) orow[j + 2] = acc4.z;
-      }
-    }
-  };
-  const bool vec_ok = (out_stride % 4 == 0) && ((uintptr_t)out % 16 == 0);
-  auto put1 = [&](int i, float v) {  // unaligned output: element stores
-    const int64_t j = jlo + i;
-    if (j < V) orow[j] = v;
-  };
-  if (mode == M_SKIP || mode == M_GREEDY || mode == M_LIST) {
-    int n = 0;
-    if (mode == M_LIST) {
-      n = rs.nlist;
-      for (int i = tid; i < n; i += CT) lst[i] = P.lists[r * DSV_LIST_K + i];
-      __syncthreads();
-    }
-    for (int i = 0; i < FE; ++i) {
-      const int64_t j = jlo + i;
-      float v = 0.f;
-      if (mode == M_GREEDY)
-        v = j == (int64_t)rs.argmax ? 1.f : 0.f;
-      else if (mode == M_LIST)
-        for (int e = 0; e < n; ++e)
-          if ((int64_t)lst[e].id == j) {
-            v = lst[e].P;
-            if (P.raw_p) {  // the unrenormalised p: recomputed from the adjusted logit
-              float x = load_elem<DT>(row_ptr(a, r), j);
-              if (P.pbits && pen_test(P, b, j))
-                x = penalize<DT>(x, a.presence ? a.presence[b] : 0.f, a.repetition ? a.repetition[b] : 1.f);
-              v = weight_of<DT>(x, DT == DT_PROB ? 1.f : a.temperatures[b], rs.m_f, rs.invZ);
-            }
-          }
-      if (vec_ok) put(i, v); else put1(i, v);
-    }
-    return;
-  }
-  const bool pen = P.pbits != nullptr;
-  const float pres = pen && a.presence ? a.presence[b] : 0.f;
-  const float rep = pen && a.repetition ? a.repetition[b] : 1.f;
-  const float T = DT == DT_PROB ? 1.f : a.temperatures[b];
-  const char* rowp = row_ptr(a, r);
-  const bool hist = mode == M_HIST;
-  int32_t tbefore = 0;
-  // the chunks' counts of the cut key's values are in rties (merged rows, and full-histogram rows
-  // whose resolver counted them)
-  const bool ties_known = !(rs.flags & FLAG_FULL_HIST) || (rs.flags & FLAG_TIES_COUNTED);
-  if (hist && rs.ktie > 0 && rs.ktie != INT_MAX) {
-    // the cut key's values before this thread's span, in id order
-    int32_t t = 0;
-    for_span<DT, ALIGNED, CT>(P, b, rowp, c, pres, rep, [&](int, float x) { t += key_of<DT>(x) == rs.vcut; });
-    int32_t tot = 0;
-    tbefore = block_excl_scan<NW>(t, red_i, &tot);
-    if (tid == 0) {
-      int32_t before = 0;
-      if (ties_known) {
-        for (int c2 = 0; c2 < c; ++c2) before += P.rties[r * NCHK + c2];
-      } else {
-        s_before = 0;
-      }
-      if (ties_known) s_before = before;
-    }
-    if (!ties_known) {  // (rare) the earlier chunks' counts by scanning them
-      int32_t e = 0;
-      for (int c2 = 0; c2 < c; ++c2)
-        for_span<DT, ALIGNED, CT>(P, b, rowp, c2, pres, rep, [&](int, float x) { e += key_of<DT>(x) == rs.vcut; });
-      e = block_sum<NW>(e, red_i);
-      if (tid == 0) s_before = e;
-    }
-    __syncthreads();
-    tbefore += s_before;
-  }
-  int32_t seen = 0;
-  for_span<DT, ALIGNED, CT>(P, b, rowp, c, pres, rep, [&](int i, float x) {
-    float v = 0.f;
-    const uint32_t k = key_of<DT>(x);
-    const bool kept = !hist || k > rs.vcut || (k == rs.vcut && (int64_t)tbefore + seen < (int64_t)rs.ktie);
-    if (kept)
-      v = P.raw_p ? weight_of<DT>(x, T, rs.m_f, rs.invZ) : (float)dense_P<DT>(rs, T, x);
-    seen += hist && k == rs.vcut;
-    if (vec_ok) put(i, v); else put1(i, v);
-  });
-}
-
-
-// ---------------------------------------------------------------------------------------
 // k_dense_p: the target distribution written out densely (runtime/worker.py:440-508), one
 // workgroup per (row, chunk).  The chunk's values are laid out as the chunk pass loads them
 // (thread t, vector u: ids (u CT + t) n .. + n), so that a wave's loads and 16-byte stores are
 // contiguous; support-list rows write zeros with the list's values at their ids (an LDS bitmap
-// of the chunk's list ids), greedy rows the one-hot row.  Rows whose cut keeps only some of the
-// values at the cut key (when the chunks' counts of them are unknown), and unaligned outputs,
-// take the ordered path above.
+// of the chunk's list ids), greedy rows the one-hot row.  Bound by the stores, and by the waves in flight
+// under them: with a separate ordered writer inlined for partial ties it held 112 registers (four waves a
+// SIMD), so 74 (bf16) and 84: 64 x 17 bf16 nucleus rows of 151936 385 -> 349 us, 1024 top-k rows of 32000
+// 71.7 -> 68.2, unfiltered rows 274 -> 267 (unaligned ones 91.0 -> 93.4 at 1024 x 32001).
 // ---------------------------------------------------------------------------------------
 template <int DT, bool ALIGNED>
 __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t out_stride) {
@@ -3225,24 +3110,21 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
   const bool hist = mode == M_HIST;
   // a cut that keeps only the first ktie values of the cut key in id order (partial ties)
   const bool part_ties = hist && rs.ktie > 0 && rs.ktie != INT_MAX;
-  const bool vec_ok = (out_stride % 4 == 0 || (uintptr_t)orow % 4 == 0);  // (any row of floats)
-  if (!vec_ok || (part_ties && (rs.flags & FLAG_FULL_HIST) && !(rs.flags & FLAG_TIES_COUNTED))) {
-    dense_p_spans<DT, ALIGNED>(P, r, c, b, rs, mode, out, out_stride);
-    return;
-  }
   const int64_t lo = (int64_t)c * CHE, hi = lo + CHE < V ? lo + CHE : V;
   const int64_t v0 = lo / n;
-  // vector u's n values at ids j0 = (v0 + u CT + tid) n: 16-byte stores, element stores at the
+  const uint32_t ext = (uint32_t)(hi - lo);  // chunk offsets in 32 bits
+  float* oc = orow + lo;
+  // vector u's n values at offsets o0 = (u CT + tid) n: 16-byte stores, element stores at the
   // row's end
-  auto store_vec = [&](int64_t j0, const float (&x)[n]) {
-    if (j0 + n <= hi) {
+  auto store_vec = [&](uint32_t o0, const float (&x)[n]) {
+    if (o0 + n <= ext) {
 #pragma unroll
       for (int q = 0; q < n / 4; ++q)
-        *reinterpret_cast<v4f4_t*>(orow + j0 + 4 * q) = v4f_t{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+        *reinterpret_cast<v4f4_t*>(oc + o0 + 4 * q) = v4f_t{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
     } else {
 #pragma unroll
       for (int e = 0; e < n; ++e)
-        if (j0 + e < hi) orow[j0 + e] = x[e];
+        if (o0 + e < ext) oc[o0 + e] = x[e];
     }
   };
   if (mode != M_UNF && !hist) {  // skipped, greedy and support-list rows
@@ -3259,11 +3141,10 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
     }
     // No logits are read here, so the values go out as 4-float groups with a wave's lanes on
     // consecutive groups (16-byte stores a wave covers 1 KB with, where the 8-value vectors of
-    // the softmax rows take two half-filled stores).  Chunk offsets in 32 bits; a group's
-    // nonzero elements from one subtraction (greedy: the one-hot's offset, -1 for none) or one
-    // bitmap nibble (support lists), the values only then
+    // the softmax rows take two half-filled stores).  A group's nonzero elements from one subtraction
+    // (greedy: the one-hot's offset, -1 for none) or one bitmap nibble (support lists), the values
+    // only then
     constexpr int G = 4;
-    const uint32_t ext = (uint32_t)(hi - lo);
     const uint32_t oh = mode == M_GREEDY ? (uint32_t)rs.argmax - (uint32_t)lo : 0xFFFFFFFFu;
 #pragma unroll
     for (int u = 0; u < CHE / G / CT; ++u) {
@@ -3315,21 +3196,43 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
   const float rep = pen && a.repetition ? a.repetition[b] : 1.f;
   const float T = DT == DT_PROB ? 1.f : a.temperatures[b];
   const char* rowp = row_ptr(a, r);
+  if constexpr (DT == DSV_BF16) {
+    // partial ties of a full-histogram row: the earlier chunks' counts of the cut key are not in rties
+    if (__builtin_expect(part_ties && (rs.flags & FLAG_FULL_HIST), 0)) {
+      __shared__ int32_t red[NW];
+      int32_t t = 0;
+#pragma unroll 4
+      for (int64_t vi = tid; vi < v0; vi += CT) {
+        const uint4 w = load_vec_any<DT>(rowp, vi, lo);
+        const uint32_t bits = pen ? pen_bits(P, b, vi * n, n) : 0u;
+#pragma unroll
+        for (int e = 0; e < n; ++e) {
+          const float x = vec_elem<DT>(w, e);
+          t += key_of<DT>((bits >> e) & 1u ? penalize<DT>(x, pres, rep) : x) == rs.vcut;
+        }
+      }
+      t = block_sum<NW>(t, red);
+      if (tid == 0) s_before = t;
+    }
+  }
   uint4 v[CV];
-  const int64_t nfull = hi / n;
+  const uint32_t nfull = ext / n;
   if constexpr (ALIGNED) {
-    const auto rsr = buf_rsrc(rowp + lo * (16 / n), (uint32_t)((hi - lo) * (16 / n)));
+    const auto rsr = buf_rsrc(rowp + lo * (16 / n), ext * (16 / n));
 #pragma unroll
     for (int u = 0; u < CV; ++u) v[u] = buf_load16(rsr, (uint32_t)tid * 16u, (uint32_t)(u * CT * 16));
-    if (hi - lo < CHE) {  // the row's last chunk: the partial last vector element by element
-      const int64_t rel = nfull - v0;
-#pragma unroll
-      for (int u = 0; u < CV; ++u)
-        if (hi % n && u == rel / CT && tid == rel % CT) v[u] = load_vec<DT>(rowp, nfull, hi, false);
-    }
   } else {
+    const char* cp = rowp + lo * (16 / n);
 #pragma unroll
-    for (int u = 0; u < CV; ++u) v[u] = load_vec_any<DT>(rowp, v0 + (int64_t)u * CT + tid, hi);
+    for (int u = 0; u < CV; ++u) {
+      const uint32_t vi = (uint32_t)(u * CT + tid);
+      v[u] = vi < nfull ? load_any(cp, vi) : make_uint4(0u, 0u, 0u, 0u);
+    }
+  }
+  if (ext % n) {  // the row's last chunk: the partial last vector element by element
+#pragma unroll
+    for (int u = 0; u < CV; ++u)
+      if ((uint32_t)(u * CT + tid) == nfull) v[u] = load_vec<DT>(rowp, v0 + nfull, hi, false);
   }
   if (pen) {
     for (int i = tid; i < CHE / 32; i += CT) {
@@ -3356,15 +3259,15 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
     int32_t incl[CV];
 #pragma unroll
     for (int u = 0; u < CV; ++u) {
-      const int64_t j0 = (v0 + (int64_t)u * CT + tid) * n;
-      int32_t cnt = 0;  // (ids past the row, zeros of the buffer loads, do not count)
+      const uint32_t o0 = (uint32_t)((u * CT + tid) * n);
+      int32_t cnt = 0;  // (ids past the row, loaded as zeros, do not count)
 #pragma unroll
-      for (int e = 0; e < n; ++e) cnt += j0 + e < hi && key_of<DT>(vec_elem<DT>(v[u], e)) == rs.vcut ? 1 : 0;
+      for (int e = 0; e < n; ++e) cnt += o0 + e < ext && key_of<DT>(vec_elem<DT>(v[u], e)) == rs.vcut ? 1 : 0;
       incl[u] = wave_incl_scan(cnt);
       rank0[u] = incl[u] - cnt;
       if (lane == WAVE - 1) s_wt[u * NW + wid] = incl[u];
     }
-    if (tid == 0) {
+    if (tid == 0 && (DT != DSV_BF16 || !(rs.flags & FLAG_FULL_HIST))) {
       int32_t before = 0;
       for (int c2 = 0; c2 < c; ++c2) before += P.rties[r * NCHK + c2];
       s_before = before;
@@ -3392,8 +3295,8 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
     constexpr bool DIV = decltype(div_tag)::value;
 #pragma unroll
     for (int u = 0; u < CV; ++u) {
-      const int64_t j0 = (v0 + (int64_t)u * CT + tid) * n;
-      if (j0 >= hi) continue;
+      const uint32_t o0 = (uint32_t)((u * CT + tid) * n);
+      if (o0 >= ext) continue;
       float x[n];
       int32_t seen = 0;
 #pragma unroll
@@ -3406,7 +3309,7 @@ __global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t o
         const float pe = weight_of<DT>(xe, T, rs.m_f, rs.invZ);
         x[e] = kept ? (DIV ? pe / rs.S_f : pe) : 0.f;
       }
-      store_vec(j0, x);
+      store_vec(o0, x);
     }
   };
   if (!P.raw_p && (rs.mode == M_HIST || rs.norm))

@@ -349,6 +349,40 @@ def test_nucleus_cut_inside_ties_across_chunks(device, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("V,pad", [(61448, 0), (61447, 0), (20488, 8), (20481, 2)])
+def test_target_probs_flat_rows_cut_inside_ties(device, dtype, V, pad):
+    """Flat rows of coarse values (the full histogram decides the cut), cut inside a group of thousands of
+    equal values in every chunk: the kept ties are the lowest ids, whole chunks and a last one of a few
+    values, aligned rows and others.  The mass ahead of the first value removed is top_p to the rounding
+    of the probabilities (2^-24 each, relative, so 2^-23 of the mass and the test's own)."""
+    from dspine_amd.verify import target_probs
+
+    g = torch.Generator().manual_seed(V)
+    bs, T = 3, 2
+    top_p = [0.9, 0.35, 0.6]
+    x = (torch.randn(bs * T, V, generator=g) * 1.5).round().to(dtype)
+    buf = torch.zeros(bs * T, V + pad, dtype=dtype, device=device)
+    rows = buf[:, :V]
+    rows.copy_(x)
+    info = W.info_to(W.sampling_info([40.0] * bs, [0] * bs, top_p), device)
+    out = torch.full((bs * T, V + pad), -1.0, device=device)
+    got = target_probs(rows, info, bs=bs, T=T, out=out[:, :V]).cpu()
+    assert pad == 0 or bool((out[:, V:] == -1).all())
+    for r in range(bs * T):
+        v, p = x[r].double(), torch.softmax(x[r].double() / 40.0, -1)
+        kept = got[r] > 0
+        last = v[kept].min()
+        assert bool(kept[v > last].all()) and not bool(kept[v < last].any())
+        ties = kept[v == last]
+        n = int(ties.sum())
+        assert 0 < n < ties.numel() and bool(ties[:n].all())  # the group split, its lowest ids kept
+        one = float(p[v == last][0])
+        mass = float(p[kept].sum())
+        assert mass - one <= top_p[r // T] + 2.0 ** -22 and mass >= top_p[r // T] - 2.0 ** -22
+        torch.testing.assert_close(got[r][kept].double(), p[kept] / mass, rtol=1e-5, atol=0)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_build_target_probs_flashinfer_min_p(device, dtype):
     """flashinfer's min-p branch on nucleus rows (top-k off or > 64): top-p on the mass
     renormalised over the top-k, then min-p against the max (tests/ref_utils.py:79-108)."""
