@@ -141,6 +141,29 @@ def test_topk_degenerate_rows(device, k):
         _topk_check(rows.to(dtype), k, device)
 
 
+@pytest.mark.parametrize("dtype,chunks,k,spread", [
+    (torch.bfloat16, 4, 33, None), (torch.bfloat16, 4, 34, None),  # bf16 lists counted, and selected by radix
+    (torch.float32, 41, 49, None), (torch.float32, 41, 50, None),  # 2009 slots in registers, 2050 not
+    (torch.float32, 64, 5, None), (torch.float32, 65, 5, None),    # a chunk count a lane, and over
+    (torch.float32, 9, 64, (63, 7)), (torch.float32, 9, 64, (63, 8)),  # 512 candidates left, and 513
+    (torch.float32, 1, 64, None), (torch.float32, 8, 256, None), (torch.float32, 9, 256, None),
+])
+def test_topk_merge_edges(device, dtype, chunks, k, spread):
+    """Both sides of every line between the merge's counting and its radix selection; a row whose last
+    chunk holds one value, one of ties.  ``spread`` (a, b): a large values in every chunk but the last, b
+    there, so that each list's smallest is a small one and the large ones all stay."""
+    n = 20480 if dtype == torch.bfloat16 else 12288
+    V = (chunks - 1) * n + (1 if chunks > 1 and spread is None else n)
+    g = torch.Generator().manual_seed(chunks * k)
+    x = torch.rand(3, V, generator=g)
+    if spread is not None:
+        for c in range(chunks):
+            at = c * n + torch.randperm(n, generator=g)[:spread[0] if c < chunks - 1 else spread[1]]
+            x[:, at] = 10.0 + torch.rand(3, at.numel(), generator=g)
+    x[2] = (x[2] * 50).round()
+    _topk_check(x.to(dtype), k, device)
+
+
 # ------------------------------------------------------------------------------------------
 # greedy verify (config: 1 x 17 x 151936 fp32)
 # ------------------------------------------------------------------------------------------
