@@ -76,12 +76,6 @@ struct RsArgs {
 };
 
 __device__ __forceinline__ float bf(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-__device__ __forceinline__ f4 bf4(const uint16_t* p) {  // 4 bf16 (8-byte aligned)
-  const uint2 w = *reinterpret_cast<const uint2*>(p);
-  return f4{__uint_as_float(w.x << 16), __uint_as_float(w.x & 0xFFFF0000u), __uint_as_float(w.y << 16),
-            __uint_as_float(w.y & 0xFFFF0000u)};
-}
-__device__ __forceinline__ f4 ld4(const float* p) { return *reinterpret_cast<const f4*>(p); }
 __device__ __forceinline__ f4 mfma(u4 a, u4 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bh8, a), __builtin_bit_cast(bh8, b), c, 0, 0, 0);
 }

@@ -3081,13 +3081,13 @@ __global__ __launch_bounds__(FCT) void k_final(KParams P) {
 // workgroup per (row, chunk).  The chunk's values are laid out as the chunk pass loads them
 // (thread t, vector u: ids (u CT + t) n .. + n), so that a wave's loads and 16-byte stores are
 // contiguous; support-list rows write zeros with the list's values at their ids (an LDS bitmap
-// of the chunk's list ids), greedy rows the one-hot row.  Bound by the stores, and by the waves in flight
-// under them: with a separate ordered writer inlined for partial ties it held 112 registers (four waves a
-// SIMD), so 74 (bf16) and 84: 64 x 17 bf16 nucleus rows of 151936 385 -> 349 us, 1024 top-k rows of 32000
-// 71.7 -> 68.2, unfiltered rows 274 -> 267 (unaligned ones 91.0 -> 93.4 at 1024 x 32001).
+// of the chunk's list ids), greedy rows the one-hot row.  Bound by the stores: bf16 rows are held to
+// four waves a SIMD where their 74 registers allow six (64 x 17 rows of 151936 of every kind 246 us
+// against 252; rows of one kind would gain by six: nucleus 385 -> 349, top-k 219 -> 217).
 // ---------------------------------------------------------------------------------------
 template <int DT, bool ALIGNED>
-__global__ __launch_bounds__(CT) void k_dense_p(KParams P, float* out, int64_t out_stride) {
+__global__ __launch_bounds__(CT) __attribute__((amdgpu_waves_per_eu(DT == DSV_BF16 ? 4 : 5, DT == DSV_BF16 ? 4 : 5)))
+void k_dense_p(KParams P, float* out, int64_t out_stride) {
   constexpr int n = Elems<DT>::n, CV = Elems<DT>::cv, CHE = Elems<DT>::chunk;
   constexpr int NW = CT / WAVE;
   __shared__ ListEntry lst[DSV_LIST_K];
