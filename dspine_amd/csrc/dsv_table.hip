@@ -17,8 +17,8 @@
 //                 products
 //   k_rs_finish   the slices combined, divided by sqrt(mean + eps)
 //
-// What bounds it: matrix-core issue and the clock under it.  n 960, K 16, H 4096, R 512, C 1024 is 92.6
-// GFLOP of float32 products, 490 GFLOP in bf16 parts: 441 us, 1.1 PFLOP/s (the library's bf16 product
+// What bounds it: matrix-core issue and the clock under it.  n 960, K 16, H 4096, R 512, C 1024 is 98.7
+// GFLOP of float32 products, 489 GFLOP in bf16 parts: 445 us, 1.1 PFLOP/s (the library's bf16 product
 // of 8192^3 runs at 1.17 on the same card).  Float32 MFMAs (16x16x4, 154 TFLOP/s at best) took 942 us.
 // Relative error against float64: 3.5e-7 (float32 MFMAs: 5.5e-7; they round after every 4 k, these
 // after every 32).
@@ -143,8 +143,9 @@ __device__ __forceinline__ int64_t state_row(const RsArgs& A, int64_t n) {
 // ---------------------------------------------------------------------------------------
 // k_rs_message: 128 sender rows x 64 R columns of both the gate and the value (the tile's 128 left
 // rows: pg rows r0.., then pv rows r0..).  Wave (w & 1, w >> 1) has 64 senders and 32 columns of
-// each; D[4g + v][li] is column 4g + v of sender li.  A stage is 64 k deep (128 us at the sizes
-// above; 32 deep, with half the products between barriers, 139 us); the weights' parts are made while
+// each; D[4g + v][li] is column 4g + v of sender li.  A stage is 64 k deep (at the sizes above
+// 128 us where 32 deep, with half the products between barriers, took 139; 148 now in the median under the
+// profiler); the weights' parts are made while
 // staging, the next stage's loads in flight in registers.
 // ---------------------------------------------------------------------------------------
 // w_last's parts, [H, 3, R]: eight values a thread.
@@ -283,9 +284,9 @@ __global__ __launch_bounds__(256, 2) void k_rs_message(RsArgs A) {
 // (w & 1, w >> 1) has 4 units and 64 h of a TH-h tile (256 or 64: rs_plan); D[4g + v][li] is h 4g + v of
 // sender li, which two 16-h blocks at a time is the B operand of the product with the head rows.
 // A stage (32 k of the tile's w_last and message parts, 72 KB) goes from memory straight to LDS, the
-// next one into the other buffer while this one is multiplied: 320 us at the sizes above.  128-h tiles
-// of four waves with the parts of w_last made while staging through registers (two workgroups a CU)
-// took 446: the splitting, 13 spilled registers, and 1.4 times the operand traffic.
+// next one into the other buffer while this one is multiplied: 333 us at the sizes above at the least,
+// 372 in the median under the profiler.  128-h tiles of four waves with the parts of w_last made while
+// staging through registers (two workgroups a CU) took 446 (this then 320 at the least): the splitting, 13 spilled registers, and 1.4 times the operand traffic.
 // ---------------------------------------------------------------------------------------
 template <int KB, int TH>
 __global__ __launch_bounds__(2 * TH, TH == 256 && KB <= 2 ? 2 : 1) void k_rs_table(RsArgs A) {
