@@ -2227,12 +2227,12 @@ __global__ __launch_bounds__(CT, ALIGNED ? (DT == DSV_BF16 ? 7 : 6) : 5) void k_
   out.pad = 0;
 
   // the softmax partial sum (support-list rows of the step only when their top-p test needs Z)
-  if constexpr (DT == DT_PROB) {  // the chunk's mass, in float64 (values past the row: -inf)
+  if constexpr (DT == DT_PROB) {  // the chunk's mass, in float64 (values past the row: -inf; a NaN stays one)
     double st_ = 0.0;
 #pragma unroll
     for (int u = 0; u < CV; ++u) {
 #pragma unroll
-      for (int e = 0; e < n; ++e) st_ += (double)fmaxf(vec_elem<DT>(v[u], e), 0.f);
+      for (int e = 0; e < n; ++e) st_ += (double)__builtin_elementwise_maximum(vec_elem<DT>(v[u], e), 0.f);
     }
     out.s = block_sum<CT / WAVE>(st_, sd);
     reg_fence(v);
@@ -2809,8 +2809,11 @@ __global__ __launch_bounds__(CT, 4) void k_merge(KParams P) {
     fetch_q_wave<DT>(P, b, s, tests, row_ptr(a, r), mode == M_UNF || mode == M_HIST, ds, ql);
   __syncthreads();
   if constexpr (DT == DT_PROB) {
-    // a top-p of 1 or more cuts a row whose raw mass is above it
-    if (mode == M_UNF && P.top_p_raw) {
+    // a row with a NaN or an infinity is divided by its mass whatever the cut (neither the candidates nor
+    // the descent's fixed point hold them); a top-p of 1 or more cuts a row whose raw mass is above it
+    if (!P.raw_p && __ballot(lane < P.C && !(pre.cs[lane].s < INFINITY))) {
+      mode = M_UNF;
+    } else if (mode == M_UNF && P.top_p_raw) {
       double mass = 0.0;
       for (int c = 0; c < P.C; ++c) mass += pre.cs[c].s;
       if ((a.backend == DSV_BACKEND_PYTORCH ? (double)(float)mass : mass) > (double)pre.top_p) mode = M_HIST;

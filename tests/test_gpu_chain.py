@@ -487,6 +487,25 @@ def test_filter_target_probs_row_forms(device, V, backend, min_p):
             assert torch.equal(got.double(), ref.double())
 
 
+@pytest.mark.parametrize("V,at", [(997, 996), (12288, 0), (24580, 24579)])
+@pytest.mark.parametrize("k,top_p,min_p", [(0, 1.0, 0.0), (0, 0.9, 0.0), (0, 0.9, 0.05), (20, 1.0, 0.0), (20, 0.9, 0.0)])
+def test_filter_target_probs_rows_with_nan_or_inf(device, V, at, k, top_p, min_p):
+    """One NaN makes a row's mass NaN and with it every value of the row, whatever the cut; an infinity
+    leaves its row's other values at zero.  Rows beside them are as they are alone."""
+    from dspine_amd.runtime.worker import filter_target_probs
+
+    O = _O()
+    g = torch.Generator().manual_seed(V)
+    p = torch.softmax(torch.randn(4, V, generator=g) * 2.0, -1)
+    p[1, at], p[2, at] = float("nan"), float("inf")
+    info = W.sampling_info([1.0] * 4, [k] * 4, [top_p] * 4, [min_p] * 4)
+    info.is_any_greedy, info.need_top_p_sampling = False, True
+    got = filter_target_probs(p.to(device), W.info_to(info, device), 1, 4, "pytorch").cpu().view(4, V)
+    ref = O.filter_target_probs(p.clone(), info, 1, 4, "pytorch").view(4, V)
+    assert torch.isnan(ref[1]).all() and torch.isnan(ref[2, at])
+    torch.testing.assert_close(got, ref, rtol=1e-5, atol=1e-9, equal_nan=True)
+
+
 def test_softmax_temp(device):
     from dspine_amd.runtime.worker import SoftmaxTemp
 
