@@ -81,11 +81,12 @@ __device__ __forceinline__ f4 mfma(u4 a, u4 b, f4 c) {
 }
 
 // x = hi + mid + lo, each bf16 (8 significant bits, round to nearest even): exact for finite float32 of
-// 2^-110 and above (below, lo and then mid end under the smallest bf16: 16 bits are left at 2^-118, 8 at
-// 2^-126).  hi is held to the largest bf16, so that a finite x above it stays finite against a zero; an
-// infinite x is (largest, inf, finite): its product with a bf16 operand is the infinity or, against zero,
-// the NaN that it is.  (Against a second split operand it may be NaN for inf, in ref alone: an infinite
-// ref makes its dot products over its norm NaN either way.)  Two values a call, packed.
+// 2^-110 and above.  Below, lo and then mid end under the smallest bf16 (16 bits are left at 2^-118, 8 at
+// 2^-126): what is lost is under 2^-133 an operand, so it shows in a table entry only where a code or a write
+// scale of 2^100 and more multiplies it.  hi is held to the largest bf16, so that a finite x above it stays
+// finite against a zero; an infinite x is (largest, inf, finite): its product with a bf16 operand is the
+// infinity or, against zero, the NaN that it is.  (Against a second split operand it may be NaN for inf, in
+// ref alone: an infinite ref makes its dot products over its norm NaN either way.)  Two values a call, packed.
 __device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   const float top = __uint_as_float(0x7F7F0000u);  // the largest bf16
   hi = __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{__builtin_amdgcn_fmed3f(a, -top, top),
